@@ -68,6 +68,7 @@ class Plan:
         self._h = h
         self.M = None
         self._keep = None
+        self._inflight = None
 
     # -- points -------------------------------------------------------------
     def setpts(self, x, y=None, z=None):
@@ -108,6 +109,10 @@ class Plan:
             if out is None:
                 out = torch.empty(self._out_shape(), dtype=tdt, device=c.device)
             rc = getattr(self._L, f"{self._pre}_execute_dev")(self._h, c.data_ptr(), out.data_ptr())
+            # the call returns with its work queued on the plan's stream, which
+            # torch's allocator does not know: held until the plan's next call,
+            # so that their memory does not go to another plan's work meanwhile
+            self._inflight = (c, out)
         else:
             c = np.ascontiguousarray(data, dtype=self.dtype).ravel()
             if c.size != self.M * self.n_trans:
@@ -132,8 +137,9 @@ class Plan:
 
     def destroy(self):
         if getattr(self, "_h", None) and self._h.value:
-            getattr(self._L, f"{self._pre}_destroy")(self._h)
+            getattr(self._L, f"{self._pre}_destroy")(self._h)  # waits for the plan's work
             self._h = C.c_void_p()
+            self._inflight = None
 
     def __del__(self):
         try:
