@@ -1013,6 +1013,35 @@ template <typename R> struct Engine {
     std::vector<Cx<double>> twI_h;
     int twI_n = -1;
     RadixPlan rpI{};
+    // tables of the DFT kernels: twiddles of the window length, and the
+    // window's cosines over the frames
+    DevBuf twN, hann;
+    std::vector<Cx<double>> twN_h, hann_h;
+    int twN_n = -1, hann_n = -1, hann_kind = -1;
+    int64_t hann_T = -1;
+
+    void dft_twiddles(int n, hipStream_t st)
+    {
+        if (twN_n == n) return;
+        upload_twiddles<double>(twN, n, st, twN_h);
+        twN_n = n;
+    }
+    void hann_table(int64_t T, int n, int kind, hipStream_t st)
+    {
+        if (hann_T == T && hann_n == n && hann_kind == kind) return;
+        hann_h.assign((size_t)T + 1, Cx<double>{0.0, 0.0});
+        const int64_t period = kind == 1 ? n + 1 : n - 1;
+        for (int64_t t = -1; t < T && n > 1; ++t) {
+            const double a = 2.0 * M_PI * (double)((t + period) % period) / (double)period;
+            hann_h[(size_t)(t + 1)].x = std::cos(a);
+            hann_h[(size_t)(t + 1)].y = std::sin(a);
+        }
+        hann.ensure(sizeof(Cx<double>) * hann_h.size());
+        HIPCHK(hipMemcpyAsync(hann.p, hann_h.data(), sizeof(Cx<double>) * hann_h.size(), hipMemcpyHostToDevice, st));
+        hann_T = T;
+        hann_n = n;
+        hann_kind = kind;
+    }
 
     int64_t nq() const { return core.N[0] * core.N[1] * core.N[2]; }
     int64_t amp_frame_elems() const { return combine ? nq() : nq() * nact; }
@@ -1267,13 +1296,16 @@ template <typename R> struct Engine {
             launch_sqw_single<R>(p, rpT, cols, amp, twT.as<Cx<R>>(), win_d.as<double>(), r->d_qfac, d_S, d_Stot, st);
             tm.end(ev, st);
         } else if (p.n_frame == 1) {
-            // one window, T without a radix plan: one DFT recurrence per frequency
+            // one window, T without a radix plan: a DFT sum per frequency
+            dft_twiddles(p.n_int, st);
             const int ev = tm.begin(ST_REDUCE, st);
-            launch_sqw_window1<R>(p, amp, r->d_qfac, win_d.as<double>(), d_S, d_Stot, st);
+            launch_sqw_window1<R>(p, amp, r->d_qfac, win_d.as<double>(), twN.as<double2>(), d_S, d_Stot, st);
             tm.end(ev, st);
         } else {
+            dft_twiddles(p.n_int, st);
+            hann_table(T, p.n_int, p.win_kind, st);
             const int ev = tm.begin(ST_REDUCE, st);
-            launch_sqw_sliding<R>(p, amp, r->d_qfac, d_S, d_Stot, st);
+            launch_sqw_sliding<R>(p, amp, r->d_qfac, twN.as<double2>(), hann.as<double2>(), d_S, d_Stot, st);
             tm.end(ev, st);
         }
         HIPCHK(hipGetLastError());
@@ -2120,8 +2152,8 @@ struct mpsq_sqw_s {
 // all frames, no mean subtraction, Hann window of the (i + 1) / (n + 1) form,
 // norm 1 / T) and the species sums.  With a radix plan for T, one fused
 // kernel per group of blocks (FFT in LDS, per-block species sums) and a
-// fixed-order reduction of the blocks' sums; otherwise one DFT recurrence
-// per frequency (k_sqw_window1) into |FFT|^2 rows (chunks of columns within
+// fixed-order reduction of the blocks' sums; otherwise DFT sums
+// (k_sqw_window1) into |FFT|^2 rows (chunks of columns within
 // 512 MB) and k_dos_species.
 template <typename R>
 static void dos_run(const float *d_vel, int64_t T, int64_t n_tot, const int32_t *d_at_ind, int nsp, int64_t n_freq,
@@ -2186,6 +2218,9 @@ static void dos_run(const float *d_vel, int64_t T, int64_t n_tot, const int32_t 
     }
     const int64_t chunk = std::max<int64_t>(1, std::min<int64_t>(ncs, ((int64_t)512 << 20) / (8 * n_f)));
     S.ensure(sizeof(double) * (size_t)(n_f * chunk));
+    DevBuf twd;
+    std::vector<Cx<double>> twdh;
+    upload_twiddles<double>(twd, (int)T, st, twdh);
     if (sizeof(R) == 8) buf.ensure(sizeof(double2) * (size_t)(T * chunk));
     for (int64_t c0 = 0; c0 < ncs; c0 += chunk) {
         const int64_t nc = std::min(chunk, ncs - c0);
@@ -2203,7 +2238,7 @@ static void dos_run(const float *d_vel, int64_t T, int64_t n_tot, const int32_t 
             launch_sqw_single<R>(p, rp, cols, amp, tw.as<Cx<R>>(), win.as<double>(), nullptr, S.as<double>(), nullptr,
                                  st);
         else
-            launch_sqw_window1<R>(p, amp, nullptr, win.as<double>(), S.as<double>(), nullptr, st);
+            launch_sqw_window1<R>(p, amp, nullptr, win.as<double>(), twd.as<double2>(), S.as<double>(), nullptr, st);
         launch_dos_species(S.as<double>(), nc, c0, n_freq, d_at_ind, nsp, d_dos, st);
         HIPCHK(hipGetLastError());
     }

@@ -8,13 +8,12 @@
 //                LDS columns, and writes |X(m)|^2 in FP64
 //                (mp_sqom56.f90:1177-1185, 1381-1387, 1480-1517, 1527, 1576).
 // k_sqw_sliding  sliding windows with hop 1 (n_frame = T - n_int + 1 > 1),
-//                any n_int: the Hann window is a sum of three exponentials,
-//                so each windowed DFT X_s(m) is a combination of three
-//                rectangular sliding DFTs that advance by an O(1) recurrence
-//                per frame (FP64); sum_s |X_s(m)|^2 accumulates in FP64
+//                any n_int: three running sums per frequency (the Hann
+//                window is a sum of three exponentials) advanced by one frame
+//                per window; sum_s |X_s(m)|^2 accumulates in FP64
 //                (mp_sqom56.f90:1437-1478 computes the same sum per energy).
 // k_sqw_window1  one window over all frames when T has no 2,3,5 radix plan:
-//                one DFT recurrence per (Q, frequency), window from a table.
+//                DFT sums of a group of frequencies per wave.
 // k_iqt          I(Q,t) (mp_sqom56.f90:1467-1471, 1504-1510) by direct sums,
 //                a thread per Q and group of lags;
 // k_iqt_fft      the same for many lags by FFT correlation in LDS (FP64).
@@ -24,6 +23,8 @@
 // k_qtables      the Q plane's q2_norm and X-ray form factor tables
 //                (mp_sqom56.f90:901-936); k_xray_table the per-Q X-ray weights
 //                of served requests on the mode grid.
+#include <algorithm>
+
 #include "mpsq_kernels.h"
 
 namespace mpsq {
@@ -140,177 +141,271 @@ __global__ __launch_bounds__(NT) void k_sqw_single(SqwParams p, RadixPlan rp, in
     }
 }
 
-// One window over all T frames (n_frame == 1) when T has no 2,3,5 radix
-// plan: thread = (Q, frequency), X(m) = sum_i w_i C'(i) e^{-2 pi i m i / n}
-// by a running twiddle with the window w from the table (one complex
-// product per frame, against three for the sliding kernel's decomposition of
-// the window into exponentials); |X|^2 and all sums in FP64.
-template <typename R>
-__global__ __launch_bounds__(256, 8) void k_sqw_window1(SqwParams p, const typename cplx<R>::T *__restrict__ amp,
-                                                     const float *__restrict__ qfac, const double *__restrict__ win,
-                                                     double *__restrict__ S, double *__restrict__ Stot)
+// Mean and sum |C|^2 of a block's 64 columns (lane = column): wave wv of nw
+// sums frames wv, wv + nw, ..., the waves' sums are added in LDS in order.
+// Every thread of the block calls it (barriers).
+template <typename A>
+__device__ __forceinline__ void column_moments(const A *__restrict__ amp, int64_t stride, int64_t T, int wv, int nw,
+                                               double (*red)[64][3], double &mr, double &mi, double &ss)
 {
+    const int lane = threadIdx.x & 63;
+    double a = 0.0, b = 0.0, c = 0.0;
+#pragma unroll 8
+    for (int64_t t = wv; t < T; t += nw) {
+        const A v = amp[t * stride];
+        a += (double)v.x;
+        b += (double)v.y;
+        c += (double)v.x * (double)v.x + (double)v.y * (double)v.y;
+    }
+    red[wv][lane][0] = a;
+    red[wv][lane][1] = b;
+    red[wv][lane][2] = c;
+    __syncthreads();
+    mr = mi = ss = 0.0;
+    for (int k = 0; k < nw; ++k) {
+        mr += red[k][lane][0];
+        mi += red[k][lane][1];
+        ss += red[k][lane][2];
+    }
+    mr /= (double)T;
+    mi /= (double)T;
+}
+
+// a += e x (four FMAs)
+__device__ __forceinline__ void cfma(double &ar, double &ai, double2 e, double xr, double xi)
+{
+    ar = __builtin_fma(e.x, xr, __builtin_fma(-e.y, xi, ar));
+    ai = __builtin_fma(e.x, xi, __builtin_fma(e.y, xr, ai));
+}
+
+// running index (m i) mod n of the frequencies' twiddles (uniform)
+__device__ __forceinline__ void step_index(int &ix, int m, int n)
+{
+    ix += m;
+    if (ix >= n) ix -= n;
+}
+
+// One window over all T frames (n_frame == 1) when T has no 2,3,5 radix
+// plan: lane = Q, wave = group of MG frequencies,
+//   X(m) = sum_i w_i C'(i) tw[(m i) mod n],  tw[k] = e^{-2 pi i k / n}.
+// The twiddles are the same for every Q, so they come from one table by
+// scalar loads and a frequency costs four FMAs per frame; a frame is read,
+// centred and windowed once per MG frequencies.  |X|^2 and all sums in FP64.
+// (A running twiddle per thread and one frequency per thread, 276,352
+// columns of 37 frames to 18 frequencies: 0.295 ms, and the map of those frames
+// fell from 2.35 to 2.15 ms with this kernel.)
+template <typename R, int MG>
+__global__ __launch_bounds__(256) void k_sqw_window1(SqwParams p, const typename cplx<R>::T *__restrict__ amp,
+                                                     const float *__restrict__ qfac, const double *__restrict__ win,
+                                                     const double2 *__restrict__ tw, double *__restrict__ S,
+                                                     double *__restrict__ Stot)
+{
+    __shared__ double red[4][64][3];
     const int64_t q = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);
-    const int mi_ = blockIdx.y * 4 + (threadIdx.x >> 6);
-    if (q >= p.NQ || mi_ >= p.n_f) return;
+    const int nw = blockDim.x >> 6, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int grp = blockIdx.y * nw + wv;
     const int n = p.n_int;
-    const int64_t qs = src_q(p, q);
-    if (qs < 0) {
-        if (mi_ == 0 && Stot) Stot[q] = qnan();
-        S[(int64_t)mi_ * p.NQ + q] = qnan();
-        return;
+    const int64_t qs = q < p.NQ ? src_q(p, q) : -1;
+    amp += qs >= 0 ? qs : 0;  // lanes without a column read column 0 and write no value of it
+    double mr = 0.0, mi = 0.0, ss = 0.0;
+    if (p.subtract_mean || Stot) column_moments(amp, p.NQs, p.T, wv, nw, red, mr, mi, ss);
+    if (q >= p.NQ || grp * MG >= p.n_f) return;
+    if (grp == 0 && Stot) Stot[q] = qs >= 0 ? ss * p.norm_tot : qnan();
+    if (!p.subtract_mean) mr = mi = 0.0;
+    int m[MG], ix[MG];
+    double dr[MG], di[MG];
+#pragma unroll
+    for (int j = 0; j < MG; ++j) {
+        const int64_t mm = (p.m_lo + (int64_t)(grp * MG + j)) % n;
+        m[j] = (int)(mm < 0 ? mm + n : mm);
+        ix[j] = 0;
+        dr[j] = di[j] = 0.0;
     }
-    amp += qs;
-    double mr = 0.0, mim = 0.0, ss = 0.0;
+#pragma unroll 4
     for (int i = 0; i < n; ++i) {
         const auto v = amp[(int64_t)i * p.NQs];
-        mr += (double)v.x;
-        mim += (double)v.y;
-        ss += (double)v.x * (double)v.x + (double)v.y * (double)v.y;
+        const double f = win[i];
+        const double cr = ((double)v.x - mr) * f, ci = ((double)v.y - mi) * f;
+#pragma unroll
+        for (int j = 0; j < MG; ++j) {
+            cfma(dr[j], di[j], tw[ix[j]], cr, ci);
+            step_index(ix[j], m[j], n);
+        }
     }
-    if (mi_ == 0 && Stot) Stot[q] = ss * p.norm_tot;
-    if (p.subtract_mean) {
-        mr /= (double)n;
-        mim /= (double)n;
-    } else {
-        mr = mim = 0.0;
+    const double qf = (qfac && qs >= 0) ? (double)qfac[qs] : 1.0;
+    const double sc = p.norm_s * qf * qf;
+#pragma unroll
+    for (int j = 0; j < MG; ++j)
+        if (grp * MG + j < p.n_f)
+            S[(int64_t)(grp * MG + j) * p.NQ + q] = qs >= 0 ? (dr[j] * dr[j] + di[j] * di[j]) * sc : qnan();
+}
+
+// Frequencies per wave of the two DFT kernels: fewest operations (a frequency
+// costs `per`, a frame's own work `fix` per wave) over the chip's 1024 SIMDs,
+// but no fewer waves than keep them busy (a wave alone waits ~50 operations
+// per frame for its loads).
+static int dft_group(int64_t NQ, int n_f, const int *sizes, int nsizes, double per, double fix)
+{
+    int best = sizes[0];
+    double bc = 1e300;
+    for (int k = 0; k < nsizes; ++k) {
+        const int mg = sizes[k];
+        const double waves = (double)((NQ + 63) / 64) * (double)((n_f + mg - 1) / mg), w = per * mg + fix;
+        const double c = std::max(waves / 1024.0 * w, w + 50.0);
+        if (c < bc) {
+            bc = c;
+            best = mg;
+        }
     }
-    const double qf = qfac ? (double)qfac[qs] : 1.0;
-    int64_t m = (p.m_lo + (int64_t)mi_) % n;
-    if (m < 0) m += n;
-    const double om = 6.283185307179586476925286766559 * (double)m / (double)n;
-    const double rr = cos(om), ri = sin(om);
-    double sr = 1.0, si = 0.0, dr = 0.0, di = 0.0;
-    for (int i = 0; i < n; ++i) {
-        const auto v = amp[(int64_t)i * p.NQs];
-        const double f = win[i] * qf;
-        const double cr = ((double)v.x - mr) * f, ci = ((double)v.y - mim) * f;
-        dr += sr * cr - si * ci;
-        di += sr * ci + si * cr;
-        const double nr = sr * rr + si * ri;  // times e^{-i om}
-        si = si * rr - sr * ri;
-        sr = nr;
-    }
-    S[(int64_t)mi_ * p.NQ + q] = (dr * dr + di * di) * p.norm_s;
+    return best;
+}
+
+// block and grid of a DFT kernel: a block holds the waves of up to 4 groups
+static void dft_launch_shape(const SqwParams &p, int mg, dim3 &grid, dim3 &block)
+{
+    const int groups = std::max(1, (p.n_f + mg - 1) / mg), nw = std::min(groups, 4);
+    grid = dim3((unsigned)((p.NQ + 63) / 64), (unsigned)((groups + nw - 1) / nw));
+    block = dim3((unsigned)(64 * nw));
 }
 
 template <typename R>
 void launch_sqw_window1(const SqwParams &p, const typename cplx<R>::T *amp, const float *qfac, const double *win,
-                        double *S, double *Stot, hipStream_t st)
+                        const double2 *tw, double *S, double *Stot, hipStream_t st)
 {
-    const unsigned gx = (unsigned)((p.NQ + 63) / 64);
-    const unsigned gy = (unsigned)((p.n_f + 3) / 4);
-    hipLaunchKernelGGL((k_sqw_window1<R>), dim3(gx, gy > 0 ? gy : 1), dim3(256), 0, st, p, amp, qfac, win, S, Stot);
+    static const int sizes[] = {1, 2, 4, 6, 8};
+    const int mg = dft_group(p.NQ, p.n_f, sizes, 5, 4.0, 6.0);
+    dim3 grid, block;
+    dft_launch_shape(p, mg, grid, block);
+#define MPSQ_WINDOW1(MG)                                                                                              \
+    case MG:                                                                                                          \
+        hipLaunchKernelGGL((k_sqw_window1<R, MG>), grid, block, 0, st, p, amp, qfac, win, tw, S, Stot);               \
+        break;
+    switch (mg) {
+        MPSQ_WINDOW1(1)
+        MPSQ_WINDOW1(2)
+        MPSQ_WINDOW1(4)
+        MPSQ_WINDOW1(6)
+        MPSQ_WINDOW1(8)
+    }
+#undef MPSQ_WINDOW1
 }
 
-// sliding windows: thread = (Q, group of MG frequencies; the launch uses 1)
+// Sliding windows (hop 1): lane = Q, wave = group of MG frequencies.  With
+// the twiddle taken at the absolute frame, tw[(m t) mod n], the window
+// w_i = (1 - cos(th (i + off))) / 2 of the frames t = s + i splits into
+//   X_s(m) e^{..} = (P - cos(th (s - off)) U - sin(th (s - off)) V) / 2,
+//   P, U, V = sum over the window of C'(t) tw (1, cos(th t), sin(th t)),
+// and advancing the window adds frame s + n and drops frame s, whose twiddles
+// are equal (n is tw's period): with d = C'(s + n) (1, c, s)(s + n) -
+// C'(s) (1, c, s)(s), formed once per frame for all MG frequencies, a
+// frequency costs 12 FMAs to advance and 6 for |X_s|^2.  Twiddles and
+// cosines are the same for every Q: scalar loads from tables made in FP64.
+// hann[t + 1] = (cos, sin)(th t), t >= -1 (zeros for n = 1, whose window is 1).
+// FP64 issue bounds it (three recurrences advanced per thread, one frequency
+// each, took 42 FMAs per window and 24 per start frame: 262,144 columns of 512
+// frames, 17 frequencies, 256 windows 6.41 ms a call, now 2.32).
 template <typename R, int MG>
-__global__ __launch_bounds__(256, 8) void k_sqw_sliding(SqwParams p, const typename cplx<R>::T *__restrict__ amp,
-                                                     const float *__restrict__ qfac, double *__restrict__ S,
+__global__ __launch_bounds__(256, 4) void k_sqw_sliding(SqwParams p, const typename cplx<R>::T *__restrict__ amp,
+                                                     const float *__restrict__ qfac, const double2 *__restrict__ tw,
+                                                     const double2 *__restrict__ hann, double *__restrict__ S,
                                                      double *__restrict__ Stot)
 {
+    __shared__ double red[4][64][3];
     const int64_t q = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);
-    const int grp = blockIdx.y * 4 + (threadIdx.x >> 6);
-    if (q >= p.NQ || grp * MG >= p.n_f) return;
-    const int64_t T = p.T;
-    const int n = p.n_int;
-    const int64_t qs = src_q(p, q);
-    if (qs < 0) {
-        if (grp == 0 && Stot) Stot[q] = qnan();
-        for (int j = 0; j < MG; ++j)
-            if (grp * MG + j < p.n_f) S[(int64_t)(grp * MG + j) * p.NQ + q] = qnan();
+    const int nw = blockDim.x >> 6, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int grp = blockIdx.y * nw + wv;
+    const int n = p.n_int, off = p.win_kind == 1 ? 1 : 0;
+    const int64_t qs = q < p.NQ ? src_q(p, q) : -1;
+    amp += qs >= 0 ? qs : 0;  // lanes without a column read column 0 and write no value of it
+    double mr, mi, ss;
+    column_moments(amp, p.NQs, p.T, wv, nw, red, mr, mi, ss);
+    if (q >= p.NQ || grp * MG >= p.n_f) {
+        if (q < p.NQ && grp == 0 && Stot) Stot[q] = qs >= 0 ? ss * p.norm_tot : qnan();
         return;
     }
-    amp += qs;
-    double mr = 0.0, mi = 0.0, ss = 0.0;
-    for (int64_t t = 0; t < T; ++t) {
-        const auto v = amp[t * p.NQs];
-        mr += (double)v.x;
-        mi += (double)v.y;
-        ss += (double)v.x * (double)v.x + (double)v.y * (double)v.y;
-    }
-    if (grp == 0 && Stot) Stot[q] = ss * p.norm_tot;
-    if (p.subtract_mean) {
-        mr /= (double)T;
-        mi /= (double)T;
-    } else {
-        mr = mi = 0.0;
-    }
-    const double qf = qfac ? (double)qfac[qs] : 1.0;
-    const double twopi = 6.283185307179586476925286766559;
-    // window = a0 + a1 e^{i th i} + a2 e^{-i th i}
-    double th = 0.0, a0 = 1.0, a1r = 0.0, a1i = 0.0;
-    if (n > 1) {
-        const int off = p.win_kind == 1 ? 1 : 0;
-        th = twopi / (double)(p.win_kind == 1 ? n + 1 : n - 1);
-        a0 = 0.5;
-        a1r = -0.25 * cos(th * off);
-        a1i = -0.25 * sin(th * off);
-    }
-    // a2 = conj(a1)
-    double Dr[MG][3], Di[MG][3], rr[MG][3], ri[MG][3], trr[MG][3], tri[MG][3], sr[MG][3], si[MG][3];
-    double acc[MG];
+    if (grp == 0 && Stot) Stot[q] = qs >= 0 ? ss * p.norm_tot : qnan();
+    if (!p.subtract_mean) mr = mi = 0.0;
+    int m[MG], ix[MG];
+    double Pr[MG], Pi[MG], Ur[MG], Ui[MG], Vr[MG], Vi[MG], acc[MG];
 #pragma unroll
     for (int j = 0; j < MG; ++j) {
-        int64_t m = (p.m_lo + (int64_t)(grp * MG + j)) % n;
-        if (m < 0) m += n;
-        const double om = twopi * (double)m / (double)n;
-        const double oms[3] = {om, om - th, om + th};
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            Dr[j][k] = Di[j][k] = 0.0;
-            rr[j][k] = cos(oms[k]);          // e^{+i w}
-            ri[j][k] = sin(oms[k]);
-            trr[j][k] = cos(oms[k] * (double)(n - 1));   // e^{-i w (n-1)}
-            tri[j][k] = -sin(oms[k] * (double)(n - 1));
-            sr[j][k] = 1.0;                  // running e^{-i w i}
-            si[j][k] = 0.0;
-        }
-        acc[j] = 0.0;
+        const int64_t mm = (p.m_lo + (int64_t)(grp * MG + j)) % n;
+        m[j] = (int)(mm < 0 ? mm + n : mm);
+        ix[j] = 0;
+        Pr[j] = Pi[j] = Ur[j] = Ui[j] = Vr[j] = Vi[j] = acc[j] = 0.0;
     }
+#pragma unroll 2
     for (int i = 0; i < n; ++i) {
         const auto v = amp[(int64_t)i * p.NQs];
-        const double cr = ((double)v.x - mr) * qf, ci = ((double)v.y - mi) * qf;
-#pragma unroll
-        for (int j = 0; j < MG; ++j)
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                Dr[j][k] += sr[j][k] * cr - si[j][k] * ci;
-                Di[j][k] += sr[j][k] * ci + si[j][k] * cr;
-                // multiply running twiddle by e^{-i w}
-                const double nr = sr[j][k] * rr[j][k] + si[j][k] * ri[j][k];
-                const double ni = si[j][k] * rr[j][k] - sr[j][k] * ri[j][k];
-                sr[j][k] = nr;
-                si[j][k] = ni;
-            }
-    }
-    for (int64_t s = 0;; ++s) {
+        const double2 h = hann[i + 1];
+        const double cr = (double)v.x - mr, ci = (double)v.y - mi;
 #pragma unroll
         for (int j = 0; j < MG; ++j) {
-            // X = a0 D0 + a1 D1 + conj(a1) D2
-            const double xr = a0 * Dr[j][0] + (a1r * Dr[j][1] - a1i * Di[j][1]) + (a1r * Dr[j][2] + a1i * Di[j][2]);
-            const double xi = a0 * Di[j][0] + (a1r * Di[j][1] + a1i * Dr[j][1]) + (a1r * Di[j][2] - a1i * Dr[j][2]);
-            acc[j] += xr * xr + xi * xi;
+            const double2 e = tw[ix[j]];
+            const double yr = e.x * cr - e.y * ci, yi = e.x * ci + e.y * cr;
+            Pr[j] += yr;
+            Pi[j] += yi;
+            Ur[j] = __builtin_fma(h.x, yr, Ur[j]);
+            Ui[j] = __builtin_fma(h.x, yi, Ui[j]);
+            Vr[j] = __builtin_fma(h.y, yr, Vr[j]);
+            Vi[j] = __builtin_fma(h.y, yi, Vi[j]);
+            step_index(ix[j], m[j], n);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < MG; ++j) ix[j] = 0;
+    for (int64_t s = 0;; ++s) {
+        const double2 a = hann[s - off + 1];
+#pragma unroll
+        for (int j = 0; j < MG; ++j) {
+            const double xr = __builtin_fma(-a.x, Ur[j], __builtin_fma(-a.y, Vr[j], Pr[j]));
+            const double xi = __builtin_fma(-a.x, Ui[j], __builtin_fma(-a.y, Vi[j], Pi[j]));
+            acc[j] = __builtin_fma(xr, xr, __builtin_fma(xi, xi, acc[j]));
         }
         if (s + 1 >= p.n_frame) break;
         const auto vo = amp[s * p.NQs];
         const auto vn = amp[(s + n) * p.NQs];
-        const double or_ = ((double)vo.x - mr) * qf, oi = ((double)vo.y - mi) * qf;
-        const double nr_ = ((double)vn.x - mr) * qf, ni = ((double)vn.y - mi) * qf;
+        const double2 ho = hann[s + 1], hn = hann[s + n + 1];
+        const double or_ = (double)vo.x - mr, oi = (double)vo.y - mi;
+        const double nr = (double)vn.x - mr, ni = (double)vn.y - mi;
+        const double d0r = nr - or_, d0i = ni - oi;
+        const double dcr = hn.x * nr - ho.x * or_, dci = hn.x * ni - ho.x * oi;
+        const double dsr = hn.y * nr - ho.y * or_, dsi = hn.y * ni - ho.y * oi;
 #pragma unroll
-        for (int j = 0; j < MG; ++j)
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                const double ar = Dr[j][k] - or_, ai = Di[j][k] - oi;
-                Dr[j][k] = (ar * rr[j][k] - ai * ri[j][k]) + (trr[j][k] * nr_ - tri[j][k] * ni);
-                Di[j][k] = (ar * ri[j][k] + ai * rr[j][k]) + (trr[j][k] * ni + tri[j][k] * nr_);
-            }
+        for (int j = 0; j < MG; ++j) {
+            const double2 e = tw[ix[j]];
+            cfma(Pr[j], Pi[j], e, d0r, d0i);
+            cfma(Ur[j], Ui[j], e, dcr, dci);
+            cfma(Vr[j], Vi[j], e, dsr, dsi);
+            step_index(ix[j], m[j], n);
+        }
     }
+    const double qf = (qfac && qs >= 0) ? (double)qfac[qs] : 1.0, wf = n > 1 ? 0.5 : 1.0;
+    const double sc = p.norm_s * (qf * qf) * (wf * wf);
 #pragma unroll
-    for (int j = 0; j < MG; ++j) {
-        const int mi_ = grp * MG + j;
-        if (mi_ < p.n_f) S[(int64_t)mi_ * p.NQ + q] = acc[j] * p.norm_s;
+    for (int j = 0; j < MG; ++j)
+        if (grp * MG + j < p.n_f) S[(int64_t)(grp * MG + j) * p.NQ + q] = qs >= 0 ? acc[j] * sc : qnan();
+}
+
+template <typename R>
+void launch_sqw_sliding(const SqwParams &p, const typename cplx<R>::T *amp, const float *qfac, const double2 *tw,
+                        const double2 *hann, double *S, double *Stot, hipStream_t st)
+{
+    static const int sizes[] = {1, 2, 3, 4};  // 4: 128 registers, four waves per SIMD
+    const int mg = dft_group(p.NQ, p.n_f, sizes, 4, 18.0, 18.0);
+    dim3 grid, block;
+    dft_launch_shape(p, mg, grid, block);
+#define MPSQ_SLIDING(MG)                                                                                              \
+    case MG:                                                                                                          \
+        hipLaunchKernelGGL((k_sqw_sliding<R, MG>), grid, block, 0, st, p, amp, qfac, tw, hann, S, Stot);              \
+        break;
+    switch (mg) {
+        MPSQ_SLIDING(1)
+        MPSQ_SLIDING(2)
+        MPSQ_SLIDING(3)
+        MPSQ_SLIDING(4)
     }
+#undef MPSQ_SLIDING
 }
 
 // Per-Q X-ray weights of nsp species on the mode grid (CMCL order, k1
@@ -808,31 +903,16 @@ void launch_sqw_single(const SqwParams &p, const RadixPlan &rp, int cols, const 
                        make_fdiv((uint32_t)p.T), amp, tw, win, qfac, S, Stot);
 }
 
-template <typename R>
-void launch_sqw_sliding(const SqwParams &p, const typename cplx<R>::T *amp, const float *qfac, double *S,
-                        double *Stot, hipStream_t st)
-{
-    // one frequency per thread, at most 64 registers (8 waves per SIMD): the
-    // recurrences of a frequency hold 36 FP64 values, so more frequencies per
-    // thread cost occupancy (a 2.1 M mode map at 17 frequencies, 256
-    // windows: 137.7 ms with 4 per thread, 87.1 with 2, 77.0 with 1 at 116
-    // registers, 50.5 with 1 at 64)
-    constexpr int MG = 1;
-    const unsigned gx = (unsigned)((p.NQ + 63) / 64);
-    const unsigned gy = (unsigned)((p.n_f + 4 * MG - 1) / (4 * MG));
-    hipLaunchKernelGGL((k_sqw_sliding<R, MG>), dim3(gx, gy > 0 ? gy : 1), dim3(256), 0, st, p, amp, qfac, S, Stot);
-}
-
 #define MPSQ_SQW_INST(R)                                                                                              \
     template int sqw_tile_elems<R>();                                                                                 \
     template size_t sqw_single_lds<R>(int64_t, int);                                                                  \
     template void launch_sqw_single<R>(const SqwParams &, const RadixPlan &, int, const cplx<R>::T *,                \
                                        const cplx<R>::T *, const double *, const float *, double *, double *,        \
                                        hipStream_t);                                                                  \
-    template void launch_sqw_sliding<R>(const SqwParams &, const cplx<R>::T *, const float *, double *, double *,    \
-                                        hipStream_t);                                                                 \
+    template void launch_sqw_sliding<R>(const SqwParams &, const cplx<R>::T *, const float *, const double2 *,       \
+                                        const double2 *, double *, double *, hipStream_t);                                                                \
     template void launch_sqw_window1<R>(const SqwParams &, const cplx<R>::T *, const float *, const double *,        \
-                                        double *, double *, hipStream_t);                                             \
+                                        const double2 *, double *, double *, hipStream_t);                                            \
     template void launch_iqt<R>(const SqwParams &, const cplx<R>::T *, const float *, double *, double *, hipStream_t); \
     template void launch_iqt_fft<R>(const SqwParams &, const RadixPlan &, int, const cplx<R>::T *, const double2 *,  \
                                     const float *, double *, double *, hipStream_t);                                 \
