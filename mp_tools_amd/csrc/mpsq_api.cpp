@@ -405,12 +405,10 @@ template <typename R> struct Core {
     bool own_stream = false;
     int warn = 0;
     int sort_chunk = 0;
-    // FP32 with real strengths: the narrow spread kernel's real form, whose
-    // 32-bit cells and paired-row x FFT allow tiles of twice the rows
+    // real strengths: the spread kernels' real forms, whose cells of half the
+    // size and paired-row x FFT allow tiles of twice the rows, and the half
+    // spectrum through the column passes
     bool real = false;
-    // real strengths (either precision): the half spectrum through the
-    // column passes
-    bool real_str = false;
     int rows_max = 1;
 
     void setup(int dim_, const int64_t *nm, int iflag_, double eps_, const mpsq_opts *o, bool real_ = false)
@@ -461,8 +459,7 @@ template <typename R> struct Core {
         // spread tile: whole x extent x (by x bz) rows within the LDS tile;
         // by + w <= n2 and bz + w <= n3 keep the rows a kernel stencil has in
         // one tile contiguous
-        real_str = real_;
-        real = real_ && sizeof(R) == 4;
+        real = real_;
         // real strengths: up to 32 rows where the complex kernel's registers
         // stop short of that (n1 = 512: 16 -> 32); grids that already allow
         // 32 rows or more keep their cap, since taller tiles of dense inputs
@@ -492,7 +489,7 @@ template <typename R> struct Core {
                 }
         }
         if (o->tile_by <= 0 && o->tile_bz <= 0) {
-            const TuneKey key{{dim, (int)n[0], (int)n[1], (int)n[2], w, sizeof(R) == 8 ? 1 : (real ? 2 : 0)}};
+            const TuneKey key{{dim, (int)n[0], (int)n[1], (int)n[2], w, (sizeof(R) == 8 ? 1 : 0) + (real ? 2 : 0)}};
             std::lock_guard<std::mutex> lk(g_tune_mu);
             auto it = g_tuned.find(key);
             if (it != g_tuned.end()) {
@@ -503,7 +500,9 @@ template <typename R> struct Core {
         if (o->tile_by > 0 && dim >= 2 && n[1] % o->tile_by == 0) by = o->tile_by;
         if (o->tile_bz > 0 && dim >= 3 && n[2] % o->tile_bz == 0) bz = o->tile_bz;
         if (by * bz > rows_max || by > bmax || bz > bmax) throw Err{MPSQ_ERR_BAD_ARG};
-        if (spread_lds<R>(by * bz, (int)n[0], w, real) > 156 * 1024) throw Err{MPSQ_ERR_SIZE};
+        if (spread_lds<R>(by, bz, (int)n[0], w, real) > 156 * 1024 ||
+            (real && sizeof(R) == 4 && spread_lds_real(by * bz, (int)n[0], w) > 156 * 1024))
+            throw Err{MPSQ_ERR_SIZE};
         if ((dim >= 2 && by + w > n[1]) || (dim >= 3 && bz + w > n[2])) throw Err{MPSQ_ERR_BAD_ARG};
         g.by = by;
         g.bz = bz;
@@ -639,7 +638,13 @@ template <typename R> struct Core {
     size_t spread_lds_size() const
     {
         const int by = (dim >= 2) ? g.by : 1, bz = (dim >= 3) ? g.bz : 1;
-        return spread_lds<R>(by * bz, g.n1, g.w, real);
+        return spread_lds<R>(by, bz, g.n1, g.w, real_launch());
+    }
+    // the tile takes the kernels of real strengths
+    bool real_launch() const
+    {
+        const int by = (dim >= 2) ? g.by : 1, bz = (dim >= 3) ? g.bz : 1;
+        return real && spread_real_ok<R>(by * bz);
     }
     SpreadJob<R> spreadjob(int ntr, const PtRec<R> *srec, int64_t nrec, int *err, const Cx<R> *cs, int64_t c_tstride,
                            const int64_t *bstart, const int *bmax, int bin_tstride, Cx<R> *G1, const float *amax,
@@ -666,14 +671,14 @@ template <typename R> struct Core {
         J.ntiles = ntiles();
         J.tile0 = 0;
         const int by = (dim >= 2) ? g.by : 1, bz = (dim >= 3) ? g.bz : 1;
-        J.grp = spread_group_rows<R>(by * bz, g.n1);
-        J.grp_sh = ilog2_ceil(J.grp);
+        J.grp = spread_group_rows<R>(by, bz, g.n1, real_launch());
+        J.npass = by * bz / J.grp;
         J.dntr = make_fdiv((uint32_t)ntr);
         J.dnt = make_fdiv((uint32_t)J.ntiles);
         J.tmajor = 0;
         J.dnty = make_fdiv((uint32_t)((dim >= 2) ? g.n2 / by : 1));
         J.dby = make_fdiv((uint32_t)by);
-        J.lds_tw = (int)spread_lds_twiddles<R>(by * bz, g.n1, g.w, real);
+        J.lds_tw = (int)spread_lds_twiddles<R>(by, bz, g.n1, g.w, real_launch());
         J.g1_len = g.N1;
         J.g1_keep = g.N1;
         return J;
@@ -1359,11 +1364,8 @@ static void run_parts(const std::vector<Part<R>> &parts, Workspace<R> &ws, Arena
     std::vector<char> real_ok(np), herm(np);
     for (int q = 0; q < np; ++q) {
         const Core<R> &c = parts[q].e->core;
-        const int rows = ((c.dim >= 2) ? c.g.by : 1) * ((c.dim >= 3) ? c.g.bz : 1);
-        real_ok[q] = c.real && spread_real_ok(rows, c.g.n1, c.g.w);
-        // FP32: only jobs of the real narrow form (the complex narrow kernel
-        // writes whole rows); FP64: the wide kernel keeps the half itself
-        herm[q] = (sizeof(R) == 8 ? c.real_str : real_ok[q]) && !part_wtab(q);
+        real_ok[q] = c.real_launch();
+        herm[q] = real_ok[q] && !part_wtab(q);
     }
     auto tpf = [&](int q) { return merged[q] ? 1 : parts[q].e->nact; };  // transforms per frame
     for (int q = 0; q < np; ++q) {
@@ -1471,7 +1473,8 @@ static void run_parts(const std::vector<Part<R>> &parts, Workspace<R> &ws, Arena
         int w;
         size_t o_jobs, o_t0, o_xr, lds;
         int njobs;
-        size_t lds_real;  // > 0: the real narrow kernel (FP32, every job's strengths real)
+        bool real;        // the kernels of real strengths, with
+        size_t lds_real;  // the LDS of the narrow one (FP32)
     };
     std::vector<SpreadLaunch> sl;
     int max_tiles = 0;  // tiles of the largest spread launch
@@ -1482,14 +1485,14 @@ static void run_parts(const std::vector<Part<R>> &parts, Workspace<R> &ws, Arena
         std::vector<int> ntl;
         int tile = 0;
         size_t lds = 0, lds_real = 0;
-        bool real = sizeof(R) == 4;
+        bool real = true;
         for (int q = 0; q < np; ++q) {
             const Engine<R> &e = *parts[q].e;
             const Core<R> &c = e.core;
             if (sclass(q) != widths[wi]) continue;
             const int rows = ((c.dim >= 2) ? c.g.by : 1) * ((c.dim >= 3) ? c.g.bz : 1);
             real = real && real_ok[q];
-            if (real) lds_real = std::max(lds_real, spread_lds_real(rows, c.g.n1, c.g.w));
+            if (real && sizeof(R) == 4) lds_real = std::max(lds_real, spread_lds_real(rows, c.g.n1, c.g.w));
             const int ntr = parts[q].b * tpf(q);
             SpreadJob<R> J = c.spreadjob(ntr, ws.srec.template as<PtRec<R>>(), npts, ws.bad.template as<int>(),
                                          ws.cs.template as<Cx<R>>(), 0,
@@ -1509,7 +1512,7 @@ static void run_parts(const std::vector<Part<R>> &parts, Workspace<R> &ws, Arena
             lds = std::max(lds, c.spread_lds_size());
         }
         sxr[wi] = xcd_ranges(cost, ntl);
-        sl.push_back(SpreadLaunch{(widths[wi] % 4096) / 16, 0, 0, 0, lds, (int)sjobs[wi].size(), real ? lds_real : 0});
+        sl.push_back(SpreadLaunch{(widths[wi] % 4096) / 16, 0, 0, 0, lds, (int)sjobs[wi].size(), real, lds_real});
         max_tiles = std::max(max_tiles, tile);
     }
     ws.fbl.ensure(sizeof(int) * (size_t)spread_max_wide_passes() * (size_t)std::max(max_tiles, 1));
@@ -1584,7 +1587,7 @@ static void run_parts(const std::vector<Part<R>> &parts, Workspace<R> &ws, Arena
     ev = tm->begin(ST_SPREAD, st);
     for (const SpreadLaunch &L : sl)
         launch_spread_jobs<R>(A.dev<SpreadJob<R>>(L.o_jobs), A.dev<int>(L.o_t0), L.njobs, L.w, A.dev<int>(L.o_xr),
-                              ws.wc.template as<int>(), ws.fbl.template as<int>(), L.lds, st, L.lds_real);
+                              ws.wc.template as<int>(), ws.fbl.template as<int>(), L.lds, st, L.real, L.lds_real);
     tm->end(ev, st);
     if (cyn > 0) {
         ev = tm->begin(ST_COLPASS, st);
@@ -1801,7 +1804,7 @@ static int autotune_impl(const mpsq_sqw_spec *spec, const float *d_pos, int64_t 
             if (by * bz > c.rows_max) continue;
             if (dim >= 2 && (n2 % by || by + w > n2)) continue;
             if (dim >= 3 && (n3 % bz || bz + w > n3)) continue;
-            if (spread_lds<R>(by * bz, n1, w, c.real) > 156 * 1024) continue;
+            if (spread_lds<R>(by, bz, n1, w, c.real) > 156 * 1024) continue;
             mpsq_sqw_spec sj = *spec;
             sj.opts.tile_by = by;
             sj.opts.tile_bz = bz;
@@ -1832,7 +1835,7 @@ static int autotune_impl(const mpsq_sqw_spec *spec, const float *d_pos, int64_t 
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     {
-        const TuneKey key{{dim, n1, n2, n3, w, sizeof(R) == 8 ? 1 : (c.real ? 2 : 0)}};
+        const TuneKey key{{dim, n1, n2, n3, w, (sizeof(R) == 8 ? 1 : 0) + (c.real ? 2 : 0)}};
         std::lock_guard<std::mutex> lk(g_tune_mu);
         g_tuned[key] = std::make_pair(bb[0], bb[1]);
     }

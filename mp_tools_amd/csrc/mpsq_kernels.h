@@ -134,7 +134,7 @@ template <typename R> struct SpreadJob {
     const float *amax;                   // per transform, or nullptr (strengths bounded by amax_s)
     float amax_s;
     const int *binmax;                   // FP32: per-bin covering bound, indexed like binstart (or nullptr)
-    int grp, grp_sh;                     // rows per x-FFT group (a power of two) and its log2
+    int grp, npass;                      // rows per wide pass, passes of a tile
     int final_conj;
     int ntr, ntiles, tile0;
     int tmajor;                          // tile ids transform-major (else position-major)
@@ -200,18 +200,18 @@ int spread_max_runs();
 int spread_max_tile_b();
 // wide passes a queued FP32 tile can take (entries of fbl per tile)
 int spread_max_wide_passes();
-// largest tile (rows of the whole x extent) of a fine grid of n1 cells in x,
-// and the rows one x-FFT group of such a tile holds
+// largest tile (rows of the whole x extent) of a fine grid of n1 cells in x
 template <typename R> int spread_max_rows(int n1);
-template <typename R> int spread_group_rows(int rows, int n1);
-// (real: the geometry of a real-strength plan, whose narrow tiles have 4-byte cells)
-template <typename R> size_t spread_lds(int rows, int n1, int w, bool real = false);
-// byte offset of the twiddles in a spread workgroup's dynamic LDS
-template <typename R> size_t spread_lds_twiddles(int rows, int n1, int w, bool real = false);
-// FP32 tiles of real strengths: whether a geometry can take the real narrow
-// kernel (rows in pairs, one 32-bit cell per row cell, two rows per complex
-// x FFT) and that kernel's dynamic LDS
-bool spread_real_ok(int rows, int n1, int w);
+// and the rows of one wide pass of a by x bz tile (real: of real strengths)
+template <typename R> int spread_group_rows(int by, int bz, int n1, bool real);
+// dynamic LDS of the launches of complex strengths, or (real) of the wide
+// launch of real ones, and the byte offset of the twiddles in it
+template <typename R> size_t spread_lds(int by, int bz, int n1, int w, bool real);
+template <typename R> size_t spread_lds_twiddles(int by, int bz, int n1, int w, bool real);
+// whether a tile of real strengths can take the real kernels (FP32: the
+// narrow one has one 32-bit cell per row cell and two rows per complex x FFT,
+// so rows come in pairs) and the FP32 narrow kernel's dynamic LDS
+template <typename R> bool spread_real_ok(int rows);
 size_t spread_lds_real(int rows, int n1, int w);
 // binmax[bs0 + b] = largest number of bin b's points whose first kernel cell
 // lies in 3 cyclically consecutive x segments (a bound on how many of them
@@ -230,14 +230,13 @@ template <typename R> int colfft_final_small_elems();
 // tiles too dense for 32-bit accumulation are queued in fbl
 // (spread_max_wide_passes() ints per tile of the table) and run by a second,
 // 64-bit launch.  All jobs share the
-// kernel width w; lds = max over jobs of spread_lds.  lds_real > 0 (FP32
-// only): every job's strengths are real (imaginary parts exactly zero; a
-// point with a nonzero one raises err) and every job's geometry passes
-// spread_real_ok, and the narrow launch takes the real form with lds_real =
-// max over jobs of spread_lds_real.
+// kernel width w; lds = max over jobs of spread_lds.  real: every job's
+// strengths are real (imaginary parts exactly zero; a point with a nonzero
+// one raises err), every job's geometry passes spread_real_ok, and
+// lds_real = max over jobs of spread_lds_real (FP32).
 template <typename R>
 void launch_spread_jobs(const SpreadJob<R> *jobs, const int *tile0s, int njobs, int w, const int *xr, int *wc,
-                        int *fbl, size_t lds, hipStream_t st, size_t lds_real = 0);
+                        int *fbl, size_t lds, hipStream_t st, bool real = false, size_t lds_real = 0);
 // |Q| histogram of partial intensities (mp_sql's Gauss integration)
 struct SqlGeom {
     int N[3];

@@ -72,7 +72,7 @@ template <> struct SpreadCfg<double> { static constexpr int E = 8, NT = 512; };
 struct NarrowCfg {
     static constexpr int E = 8, NT = 512;
 };
-constexpr int MAX_WIDE_PASSES = 8;  // narrow tile rows / wide pass rows (32-row real tiles: 8)
+constexpr int MAX_WIDE_PASSES = 16;  // wide passes of a tile (a tile has at most twice the rows one pass holds)
 
 constexpr int MAX_TILE_B = 16;   // by, bz <= 16
 constexpr int NARROW_MAX = 256;  // largest covering bound of a 32-bit (narrow) FP32 tile
@@ -139,7 +139,8 @@ __device__ __forceinline__ void overlap(int l, int r0, int b, int w, int n, int 
 //   narrow cells  packed 8-byte cells of row r at [r * RSX, r * RSX + RS),
 //                 counted from byte narrow_bias(w) (so that a lane's base
 //                 address minus 8w is never negative, see k_spread_narrow);
-//   wide planes   one pass of G rows: [2][G][RS] 8-byte cells;
+//   wide planes   one pass of G rows: [2][G][RS] 8-byte cells, or one plane
+//                 of twice the rows where the strengths are real;
 // then the n1 twiddles.
 __host__ __device__ inline int spread_row_stride(int n1, int w) { return (n1 + w + 1) & ~1; }
 __host__ __device__ inline int spread_row_stride_x(int n1, int w)
@@ -154,30 +155,41 @@ template <typename R> int spread_max_rows(int n1)
     while (2 * g * n1 <= te) g *= 2;
     return g;
 }
-template <typename R> int spread_group_rows(int rows, int n1)
+// Rows of one wide pass of a by x bz tile: the most that the x FFT's registers
+// take (real strengths: rows in pairs, so twice as many), as whole z planes
+// of the tile or, where one plane is too many, an equal part of a plane -- a
+// pass is a rectangle of the tile, with candidates of its own.
+template <typename R> int spread_group_rows(int by, int bz, int n1, bool real)
 {
-    const int te = SpreadCfg<R>::E * SpreadCfg<R>::NT;
-    int g = 1;
-    while (2 * g <= rows && 2 * g * n1 <= te) g *= 2;
-    return g;
+    const int te = SpreadCfg<R>::E * SpreadCfg<R>::NT * (real ? 2 : 1);
+    auto fits = [&](int g) { return (real ? (g + 1) / 2 * 2 : g) * n1 <= te; };
+    for (int k = bz; k >= 1; --k)
+        if (bz % k == 0 && fits(by * k)) return by * k;
+    for (int k = by - 1; k > 1; --k)
+        if (by % k == 0 && fits(k)) return k;
+    return 1;
 }
 // bytes of the tile region (accumulators / FFT rows); the twiddles follow it
-// (real: the narrow kernel's real form, 4-byte cells)
 __host__ __device__ constexpr int narrow_bias(int w) { return (8 * w + 15) / 16 * 16; }
-template <typename R> size_t spread_tile_bytes(int rows, int n1, int w, bool real = false)
+template <typename R> size_t spread_tile_bytes(int by, int bz, int n1, int w, bool real)
 {
-    const size_t G = (size_t)spread_group_rows<R>(rows, n1);
-    const size_t RSX = (size_t)spread_row_stride_x(n1, w);
-    const size_t narrowb = sizeof(R) == 4 ? (size_t)rows * RSX * (real ? 4 : 8) + (size_t)narrow_bias(w) : 0;
-    const size_t wideb = std::max(2 * G * spread_row_stride(n1, w) * 8, G * RSX * sizeof(typename cplx<R>::T));
+    const size_t rows = (size_t)by * bz, G = (size_t)spread_group_rows<R>(by, bz, n1, real);
+    const size_t RS = (size_t)spread_row_stride(n1, w), RSX = (size_t)spread_row_stride_x(n1, w);
+    const size_t cb = sizeof(typename cplx<R>::T);
+    if (real) {  // a wide pass of the real form: one 8-byte cell per row cell, FFT rows per pair
+        const size_t pairs = (G + 1) / 2;
+        return (std::max(2 * pairs * RS * 8, pairs * RSX * cb) + 15) / 16 * 16;
+    }
+    const size_t narrowb = sizeof(R) == 4 ? rows * RSX * 8 + (size_t)narrow_bias(w) : 0;
+    const size_t wideb = std::max(2 * G * RS * 8, G * RSX * cb);
     return (std::max(narrowb, wideb) + 15) / 16 * 16;
 }
-template <typename R> size_t spread_lds_bytes(int rows, int n1, int w, bool real = false)
+template <typename R> size_t spread_lds_bytes(int by, int bz, int n1, int w, bool real)
 {
-    // + n1 twiddles; FP32: + the tile's scaled deconvolution factors (N1 <= n1 / 2
+    // + n1 twiddles; narrow: + the tile's scaled deconvolution factors (N1 <= n1 / 2
     // floats) and its rows' output offsets (rows int64)
-    const size_t extra = sizeof(R) == 4 ? (size_t)(n1 / 2) * 4 + (size_t)rows * 8 : 0;
-    return spread_tile_bytes<R>(rows, n1, w, real) + (size_t)n1 * sizeof(typename cplx<R>::T) + extra;
+    const size_t extra = (sizeof(R) == 4 && !real) ? (size_t)(n1 / 2) * 4 + (size_t)by * bz * 8 : 0;
+    return spread_tile_bytes<R>(by, bz, n1, w, real) + (size_t)n1 * sizeof(typename cplx<R>::T) + extra;
 }
 // byte offset of the narrow kernel's per-tile tables after the twiddles
 __host__ __device__ inline int spread_tab_offset(int lds_tw, int n1) { return lds_tw + n1 * 8; }
@@ -439,6 +451,7 @@ __device__ __forceinline__ void tile_decode(const SpreadJob<R> &J, int id, int &
 struct RunTable {
     int64_t rbeg[2][MAX_RUNS];
     int rpre[2][MAX_RUNS + 1];
+    int nruns[2];
     float amax[2];
     int cb[2];
     int next;
@@ -448,12 +461,12 @@ struct RunTable {
 // the sizes), its strength bound and, with `bound`, its covering bound (the
 // sum of the visited bins' bounds), published in buffer pb.
 template <typename R>
-__device__ __forceinline__ void runs_publish(RunTable &S, int pb, const SpreadJob<R> &J, int t, int y0, int z0,
-                                             int lane, bool bound)
+__device__ __forceinline__ void runs_publish(RunTable &S, int pb, const SpreadJob<R> &J, int t, int y0, int z0, int by,
+                                             int bz, int lane, bool bound)
 {
     const Geo &g = J.g;
     int ylo, nyb, zlo, nzb;
-    tile_bins(g, y0, z0, ylo, nyb, zlo, nzb);
+    rect_bins(g, y0, z0, by, bz, ylo, nyb, zlo, nzb);
     const int nruns = 2 * nzb;  // <= MAX_RUNS (checked by the host)
     int64_t b0 = 0;
     int cnt = 0;
@@ -485,6 +498,7 @@ __device__ __forceinline__ void runs_publish(RunTable &S, int pb, const SpreadJo
     }
     if (lane == 0) {
         S.rpre[pb][0] = 0;
+        S.nruns[pb] = nruns;
         S.amax[pb] = J.amax ? J.amax[t] : J.amax_s;
         S.cb[pb] = cb;
     }
@@ -520,10 +534,9 @@ template <typename R> struct Cand {
     }
 };
 
-// kept frequency f of tile row r, times 2^e2 / phi_hat (conjugated if asked), to G1
+// kept frequency f of grid row (y, z), times 1 / phi_hat (conjugated if asked), to G1
 template <typename R>
-__device__ __forceinline__ void store_kept(const SpreadJob<R> &J, int t, int y0, int z0, int by, int r, int f,
-                                           typename cplx<R>::T v, int e2)
+__device__ __forceinline__ void store_kept(const SpreadJob<R> &J, int t, int y, int z, int f, typename cplx<R>::T v)
 {
     const Geo &g = J.g;
     const int N1 = g.N1, h1 = N1 / 2, n1 = g.n1;
@@ -533,10 +546,8 @@ __device__ __forceinline__ void store_kept(const SpreadJob<R> &J, int t, int y0,
     else return;
     if (kk >= J.g1_keep) return;  // half spectrum: k1 <= 0 only
     v = cscale(v, J.phinv1[kk]);
-    if (e2) v = cmk<typename cplx<R>::T>(ldexp(v.x, e2), ldexp(v.y, e2));
     if (J.final_conj) v.y = -v.y;
-    const int rz = (int)fdiv((uint32_t)r, J.dby), ry = r - rz * by;
-    J.G1[(((int64_t)t * g.n3 + z0 + rz) * g.n2 + y0 + ry) * J.g1_len + kk] = v;
+    J.G1[(((int64_t)t * g.n3 + z) * g.n2 + y) * J.g1_len + kk] = v;
 }
 
 template <typename R, int NT>
@@ -628,12 +639,14 @@ __global__ __launch_bounds__(NarrowCfg::NT, 4) void k_spread_narrow(const Spread
     tile_decode(jobs[j], cur, t, y0, z0);
     load_twiddles<R, NT>(jobs[j], smem_raw, tw_off(jobs[j]));
     int pb = 0;
-    if (wv == 0) runs_publish(S, pb, jobs[j], t, y0, z0, lane, true);
+    auto rows_y = [](const Geo &gq) { return (gq.dim >= 2) ? gq.by : 1; };
+    auto rows_z = [](const Geo &gq) { return (gq.dim >= 3) ? gq.bz : 1; };
+    if (wv == 0) runs_publish(S, pb, jobs[j], t, y0, z0, rows_y(jobs[j].g), rows_z(jobs[j].g), lane, true);
     __syncthreads();
     // two candidates per lane in flight: this one and the one NT further
     Cand<R> c0, c1;
     int e = 0;
-    int total = S.rpre[pb][nruns_of(jobs[j].g, y0, z0)];
+    int total = S.rpre[pb][S.nruns[pb]];
     c0.fetch(jobs[j], S, pb, vw + lane, t, total, e);
     c1.fetch(jobs[j], S, pb, vw + NT + lane, t, total, e);
 
@@ -674,7 +687,7 @@ __global__ __launch_bounds__(NarrowCfg::NT, 4) void k_spread_narrow(const Spread
                 rowoff[r] = (((int64_t)t * g.n3 + z0 + rz) * g.n2 + y0 + ry) * J.g1_len;
             }
         } else if (threadIdx.x == 0) {
-            const int np = rows >> J.grp_sh;  // wide passes of G rows
+            const int np = J.npass;  // wide passes of J.grp rows
             const int k = atomicAdd(wc + CTR_FB_COUNT, np);
             for (int p = 0; p < np; ++p) fbl[k + p] = cur * MAX_WIDE_PASSES + p;
         }
@@ -689,7 +702,8 @@ __global__ __launch_bounds__(NarrowCfg::NT, 4) void k_spread_narrow(const Spread
                 int jq, tq, y0q, z0q;
                 jq = job_of(tile0s, njobs, nxt);
                 tile_decode(jobs[jq], nxt, tq, y0q, z0q);
-                runs_publish(S, pb ^ 1, jobs[jq], tq, y0q, z0q, lane, true);
+                runs_publish(S, pb ^ 1, jobs[jq], tq, y0q, z0q, rows_y(jobs[jq].g), rows_z(jobs[jq].g), lane,
+                             true);
             }
         }
 
@@ -780,7 +794,7 @@ __global__ __launch_bounds__(NarrowCfg::NT, 4) void k_spread_narrow(const Spread
         if (has_next) {
             jn = job_of(tile0s, njobs, nxt);
             tile_decode(jobs[jn], nxt, tn, y0n, z0n);
-            total_n = S.rpre[pb ^ 1][nruns_of(jobs[jn].g, y0n, z0n)];
+            total_n = S.rpre[pb ^ 1][S.nruns[pb ^ 1]];
             e = 0;
             c0.fetch(jobs[jn], S, pb ^ 1, vw + lane, tn, total_n, e);
             c1.fetch(jobs[jn], S, pb ^ 1, vw + NT + lane, tn, total_n, e);
@@ -893,13 +907,38 @@ __global__ __launch_bounds__(NarrowCfg::NT, 4) void k_spread_narrow(const Spread
 }
 
 // ---------------------------------------------------------------------------
-// Wide spread + x FFT: one pass of G rows of a tile per item.  Items are
-// either every tile of the table (fbl == nullptr; per-XCD ranges as in the
-// narrow kernel) or the list fbl[0 .. wc[CTR_FB_COUNT]) the narrow kernel
-// queued (item = tile id * MAX_WIDE_PASSES + pass), taken through
-// wc[CTR_FB_TAKE].
+// Wide spread + x FFT: one pass of G = J.grp rows of a tile per item.  Items
+// are either every tile of the table (fbl == nullptr; per-XCD ranges as in the
+// narrow kernel; a tile is one pass) or the list fbl[0 .. wc[CTR_FB_COUNT])
+// the narrow kernel queued (item = tile id * MAX_WIDE_PASSES + pass), taken
+// through wc[CTR_FB_TAKE].  A pass is a rectangle of the tile (whole z planes,
+// or part of one plane) and visits the candidates of that rectangle only.
+//
+// REAL: the strengths are real (the host guarantees it; a point with a nonzero
+// imaginary part is skipped and raises err).  One 8-byte cell per row cell
+// instead of two, so a pass holds twice the rows in the same LDS and a
+// contribution is one atomic; rows 2p and 2p + 1 enter one complex x FFT as re
+// and im and are split by Hermitian symmetry, as in the narrow kernel.
+// (FP64 map, 320,000 atoms x 16 frames to 256 x 256 x 32: 7.41 -> 4.49 ms a
+// call; a 10.5 M atom frame to 512 x 512 x 64 in FP32, whose tiles are all
+// queued: 9.94 -> 5.80 ms.)
 // ---------------------------------------------------------------------------
-template <typename R, int W>
+struct PassRect {
+    int y0, z0, by, bz;  // rows of the pass: by x bz from (y0, z0)
+};
+template <typename R>
+__device__ __forceinline__ PassRect pass_rect(const SpreadJob<R> &J, int y0, int z0, int pass)
+{
+    const int by = (J.g.dim >= 2) ? J.g.by : 1, G = J.grp;
+    if (G >= by) {
+        const int kz = G / by;
+        return PassRect{y0, z0 + pass * kz, by, kz};
+    }
+    const int r0 = pass * G, rz = (int)fdiv((uint32_t)r0, J.dby);
+    return PassRect{y0 + r0 - rz * by, z0 + rz, G, 1};
+}
+
+template <typename R, int W, bool REAL>
 __global__ __launch_bounds__(512, 4) void k_spread_wide(const SpreadJob<R> *__restrict__ jobs,
                                                         const int *__restrict__ tile0s, int njobs,
                                                         const int *__restrict__ xr, int *__restrict__ wc,
@@ -928,23 +967,28 @@ __global__ __launch_bounds__(512, 4) void k_spread_wide(const SpreadJob<R> *__re
         id = it / MAX_WIDE_PASSES;
         pass = it % MAX_WIDE_PASSES;
     };
+    // job, transform and rows of an item
+    auto item_rows = [&](int id, int pass, int &j, int &t) -> PassRect {
+        j = job_of(tile0s, njobs, id);
+        int y0, z0;
+        tile_decode(jobs[j], id, t, y0, z0);
+        return pass_rect(jobs[j], y0, z0, pass);
+    };
 
     if (threadIdx.x == 0) S.next = take();
     __syncthreads();
     const int kfirst = S.next;
     if (kfirst >= xend) return;
-    int cur, pass;
-    item_of(kfirst, cur, pass);
-    int j = job_of(tile0s, njobs, cur);
-    int t, y0, z0;
-    tile_decode(jobs[j], cur, t, y0, z0);
+    int id0, pass0, j, t;
+    item_of(kfirst, id0, pass0);
+    PassRect P = item_rows(id0, pass0, j, t);
     load_twiddles<R, NT>(jobs[j], smem_raw, jobs[j].lds_tw);
     int pb = 0;
-    if (wv == 0) runs_publish(S, pb, jobs[j], t, y0, z0, lane, false);
+    if (wv == 0) runs_publish(S, pb, jobs[j], t, P.y0, P.z0, P.by, P.bz, lane, false);
     __syncthreads();
     Cand<R> cd;
     int e = 0;
-    int total = S.rpre[pb][nruns_of(jobs[j].g, y0, z0)];
+    int total = S.rpre[pb][S.nruns[pb]];
     cd.fetch(jobs[j], S, pb, vw + lane, t, total, e);
 
     for (;;) {
@@ -953,18 +997,18 @@ __global__ __launch_bounds__(512, 4) void k_spread_wide(const SpreadJob<R> *__re
         const int n1 = g.n1, w = g.w;
         const int RS = spread_row_stride(n1, W);
         const int RSX = spread_row_stride_x(n1, W);
-        const int by = (g.dim >= 2) ? g.by : 1;
-        const int bz = (g.dim >= 3) ? g.bz : 1;
-        const int G = J.grp;
-        const int r0 = pass * G;    // tile rows [r0, r0 + G) of this item
+        const int G = P.by * P.bz;
         const int wplane = G * RS;  // cells of one plane
+        const int pairs = (G + 1) >> 1;
+        const int nyb = min(W, P.by);  // kernel values along y a pass can use
         const R beta = es_shape<R>(g.beta), ic = (R)g.ic;
         const C *tw = reinterpret_cast<const C *>(smem_raw + J.lds_tw);
         const float am = S.amax[pb];
 
         {
             uint4 *a4 = reinterpret_cast<uint4 *>(smem_raw);
-            for (int i = threadIdx.x; i < wplane; i += NT) a4[i] = make_uint4(0u, 0u, 0u, 0u);
+            const int n16 = REAL ? pairs * RS : wplane;
+            for (int i = threadIdx.x; i < n16; i += NT) a4[i] = make_uint4(0u, 0u, 0u, 0u);
         }
         __syncthreads();
         if (wv == 0) {
@@ -973,11 +1017,10 @@ __global__ __launch_bounds__(512, 4) void k_spread_wide(const SpreadJob<R> *__re
             kn = __shfl(kn, 0, 64);
             if (lane == 0) S.next = kn;
             if (kn < xend) {
-                int idq, pq, jq, tq, y0q, z0q;
+                int idq, pq, jq, tq;
                 item_of(kn, idq, pq);
-                jq = job_of(tile0s, njobs, idq);
-                tile_decode(jobs[jq], idq, tq, y0q, z0q);
-                runs_publish(S, pb ^ 1, jobs[jq], tq, y0q, z0q, lane, false);
+                const PassRect Q = item_rows(idq, pq, jq, tq);
+                runs_publish(S, pb ^ 1, jobs[jq], tq, Q.y0, Q.z0, Q.by, Q.bz, lane, false);
             }
         }
 
@@ -998,9 +1041,15 @@ __global__ __launch_bounds__(512, 4) void k_spread_wide(const SpreadJob<R> *__re
             const bool hv = cd.have;
             cd.fetch(J, S, pb, v0 + NT + lane, t, total, e);
             if (!hv) continue;
+            if constexpr (REAL) {
+                if (cc.y != (R)0) {  // 1 for a NaN (non-finite input), else 2
+                    atomicOr(J.err, cc.y == cc.y ? 2 : 1);
+                    continue;
+                }
+            }
             int fy = 0, ny = 1, my = 0, fz = 0, nz = 1, mz = 0;
-            if (g.dim >= 2) overlap(p.ly, y0, by, w, g.n2, fy, ny, my);
-            if (g.dim >= 3) overlap(p.lz, z0, bz, w, g.n3, fz, nz, mz);
+            if (g.dim >= 2) overlap(p.ly, P.y0, P.by, w, g.n2, fy, ny, my);
+            if (g.dim >= 3) overlap(p.lz, P.z0, P.bz, w, g.n3, fz, nz, mz);
             if (ny <= 0 || nz <= 0) continue;
             double kxd[W];
             R kx[W];
@@ -1011,26 +1060,29 @@ __global__ __launch_bounds__(512, 4) void k_spread_wide(const SpreadJob<R> *__re
             }
             R ky[W];
 #pragma unroll
-            for (int iy = 0; iy < W; ++iy)
-                ky[iy] = (g.dim >= 2) ? ((iy < ny) ? es_kernel(p.dy + (R)(my + iy), beta, ic) : (R)0) : (R)1;
+            for (int iy = 0; iy < W; ++iy) {
+                ky[iy] = (R)0;
+                if (iy < nyb)  // uniform
+                    ky[iy] = (g.dim >= 2) ? ((iy < ny) ? es_kernel(p.dy + (R)(my + iy), beta, ic) : (R)0) : (R)1;
+            }
             for (int iz = 0; iz < nz; ++iz) {
                 const R wz = (g.dim >= 3) ? es_kernel(p.dz + (R)(mz + iz), beta, ic) : (R)1;
-                const int rr0 = (fz + iz) * by + fy - r0;  // pass row of iy = 0
+                const int rr0 = __mul24(fz + iz, P.by) + fy;  // pass row of iy = 0
 #pragma unroll
                 for (int iy = 0; iy < W; ++iy) {
-                    const int r = rr0 + iy;
-                    if (iy < ny && r >= 0 && r < G) {
+                    if (iy < nyb && iy < ny) {
                         const R wyz = ky[iy] * wz;
-                        const int c0 = r * RS + p.lx;
+                        const int c0 = __mul24(rr0 + iy, RS) + p.lx;
                         if (F32) {
                             const double vr = (double)(cc.x * wyz), vi = (double)(cc.y * wyz);
                             unsigned long long *ar = acc64 + c0, *ai = acc64 + wplane + c0;
 #pragma unroll
                             for (int m = 0; m < W; ++m) {
                                 const double dr = __builtin_fma(vr, kxd[m], FIX_MAGIC);
-                                const double di = __builtin_fma(vi, kxd[m], FIX_MAGIC);
                                 __hip_atomic_fetch_add(ar + m, (unsigned long long)__double_as_longlong(dr),
                                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                                if constexpr (REAL) continue;
+                                const double di = __builtin_fma(vi, kxd[m], FIX_MAGIC);
                                 __hip_atomic_fetch_add(ai + m, (unsigned long long)__double_as_longlong(di),
                                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                             }
@@ -1041,6 +1093,7 @@ __global__ __launch_bounds__(512, 4) void k_spread_wide(const SpreadJob<R> *__re
                             for (int m = 0; m < W; ++m) {
                                 __hip_atomic_fetch_add(ar + m, (double)(vr * kx[m]), __ATOMIC_RELAXED,
                                                        __HIP_MEMORY_SCOPE_WORKGROUP);
+                                if constexpr (REAL) continue;
                                 __hip_atomic_fetch_add(ai + m, (double)(vi * kx[m]), __ATOMIC_RELAXED,
                                                        __HIP_MEMORY_SCOPE_WORKGROUP);
                             }
@@ -1052,43 +1105,77 @@ __global__ __launch_bounds__(512, 4) void k_spread_wide(const SpreadJob<R> *__re
         __syncthreads();
         const int kn = S.next;
         const bool has_next = kn < xend;
-        int nid = 0, npass = 0, jn = j, tn = 0, y0n = 0, z0n = 0, total_n = 0;
+        int jn = j, tn = 0, total_n = 0;
+        PassRect Pn{0, 0, 1, 1};
         if (has_next) {
+            int nid, npass;
             item_of(kn, nid, npass);
-            jn = job_of(tile0s, njobs, nid);
-            tile_decode(jobs[jn], nid, tn, y0n, z0n);
-            total_n = S.rpre[pb ^ 1][nruns_of(jobs[jn].g, y0n, z0n)];
+            Pn = item_rows(nid, npass, jn, tn);
+            total_n = S.rpre[pb ^ 1][S.nruns[pb ^ 1]];
             e = 0;
             cd.fetch(jobs[jn], S, pb ^ 1, vw + lane, tn, total_n, e);
         }
 
         // ---- x FFT of the item's G rows
         {
-            // the ghost cells x = n1 + i fold onto i < w here
-            auto load_acc = [&](int row, int i) -> C {
-                const int a = row * RS + i;
+            // cell a of a plane as a number (FP32: the low 48 bits of the
+            // pattern sum); the ghost cells x = n1 + i fold onto i < w here
+            auto cell = [&](int a, bool ghost) -> R {
                 if (F32) {
-                    unsigned long long ur = acc64[a], ui = acc64[wplane + a];
-                    if (i < W) {
-                        ur += acc64[a + n1];
-                        ui += acc64[wplane + a + n1];
-                    }
-                    const long long br = (long long)(ur << 16) >> 16;
-                    const long long bi = (long long)(ui << 16) >> 16;
-                    return cmk<C>(fbad ? (R)NAN : (R)((double)br * finv), fbad ? (R)NAN : (R)((double)bi * finv));
-                } else {
-                    double dr = accd[a], di = accd[wplane + a];
-                    if (i < W) {
-                        dr += accd[a + n1];
-                        di += accd[wplane + a + n1];
-                    }
-                    return cmk<C>((R)dr, (R)di);
+                    unsigned long long u = acc64[a];
+                    if (ghost) u += acc64[a + n1];
+                    return fbad ? (R)NAN : (R)((double)((long long)(u << 16) >> 16) * finv);
                 }
+                double d = accd[a];
+                if (ghost) d += accd[a + n1];
+                return (R)d;
             };
             auto load_tile = [&](int row, int i) -> C { return tile[row * RSX + padx<true>(i)]; };
             auto store_tile = [&](int row, int i, C v) { tile[row * RSX + padx<true>(i)] = v; };
-            auto store_out = [&](int row, int f, C v) { store_kept(J, t, y0, z0, by, r0 + row, f, v, 0); };
-            x_fft<C, E, NT>(J.rp1, n1, G, tw, load_acc, load_tile, store_tile, store_out);
+            // grid row of pass row r
+            auto row_y = [&](int r, int &y, int &z) {
+                const int rz = P.bz > 1 ? (int)fdiv((uint32_t)r, J.dby) : 0;
+                y = P.y0 + r - rz * P.by;
+                z = P.z0 + rz;
+            };
+            if constexpr (REAL) {
+                auto load_pair = [&](int pr, int i) -> C {
+                    const int a = 2 * pr * RS + i;
+                    return cmk<C>(cell(a, i < W), cell(a + RS, i < W));
+                };
+                x_fft<C, E, NT, true>(J.rp1, n1, pairs, tw, load_pair, load_tile, store_tile, store_tile);
+                __syncthreads();
+                // kept frequency kk of rows 2 pr and 2 pr + 1 from Z = FFT(row 2 pr + i row 2 pr + 1)
+                const int h1 = g.N1 / 2, KO = J.g1_keep;
+                for (int pr = wv; pr < pairs; pr += NT / 64) {
+                    const C *zr = tile + pr * RSX;
+                    int ya, za, yb, zb;
+                    row_y(2 * pr, ya, za);
+                    row_y(2 * pr + 1, yb, zb);
+                    C *ga = J.G1 + (((int64_t)t * g.n3 + za) * g.n2 + ya) * J.g1_len;
+                    C *gb = J.G1 + (((int64_t)t * g.n3 + zb) * g.n2 + yb) * J.g1_len;
+                    const bool two = 2 * pr + 1 < G;
+                    for (int kk = lane; kk < KO; kk += 64) {
+                        const int f = (kk >= h1) ? kk - h1 : kk + n1 - h1;
+                        const C z = zr[padx<true>(f)], y = zr[padx<true>(f == 0 ? 0 : n1 - f)];
+                        const R sc = (R)0.5 * J.phinv1[kk];
+                        const R xi = (z.y - y.y) * sc, yi = (y.x - z.x) * sc;
+                        ga[kk] = cmk<C>((z.x + y.x) * sc, J.final_conj ? -xi : xi);
+                        if (two) gb[kk] = cmk<C>((z.y + y.y) * sc, J.final_conj ? -yi : yi);
+                    }
+                }
+            } else {
+                auto load_acc = [&](int row, int i) -> C {
+                    const int a = row * RS + i;
+                    return cmk<C>(cell(a, i < W), cell(wplane + a, i < W));
+                };
+                auto store_out = [&](int row, int f, C v) {
+                    int y, z;
+                    row_y(row, y, z);
+                    store_kept(J, t, y, z, f, v);
+                };
+                x_fft<C, E, NT>(J.rp1, n1, G, tw, load_acc, load_tile, store_tile, store_out);
+            }
         }
         if (!has_next) break;
         __syncthreads();  // every read of the tile (and the twiddles) done
@@ -1096,9 +1183,7 @@ __global__ __launch_bounds__(512, 4) void k_spread_wide(const SpreadJob<R> *__re
         pb ^= 1;
         j = jn;
         t = tn;
-        y0 = y0n;
-        z0 = z0n;
-        pass = npass;
+        P = Pn;
         total = total_n;
     }
 }
@@ -1124,16 +1209,17 @@ inline int persistent_grid(const void *fn, int nt, size_t lds)
     return it->second;
 }
 
-// the narrow (FP32; real or complex strengths) and wide launches of width W
+// the narrow (FP32) and wide launches of width W, in the form for real or for
+// complex strengths
 template <typename R, int W>
 void launch_spread_w(const SpreadJob<R> *jobs, const int *tile0s, int njobs, const int *xr, int *wc, int *fbl,
-                     size_t lds, hipStream_t st, size_t lds_real)
+                     size_t lds, hipStream_t st, bool real, size_t lds_real)
 {
     constexpr int NT = SpreadCfg<R>::NT;
     launch_zero_i32(wc, XCD_CTR_INTS, st);
-    const void *fw = reinterpret_cast<const void *>(&k_spread_wide<R, W>);
+    const int *items = nullptr;  // the wide launch's items: every tile, or
     if constexpr (sizeof(R) == 4) {
-        if (lds_real > 0) {
+        if (real) {
             const void *fn = reinterpret_cast<const void *>(&k_spread_narrow<W, true>);
             hipLaunchKernelGGL((k_spread_narrow<W, true>), dim3((unsigned)persistent_grid(fn, NarrowCfg::NT, lds_real)),
                                dim3(NarrowCfg::NT), lds_real, st, jobs, tile0s, njobs, xr, wc, fbl);
@@ -1142,18 +1228,23 @@ void launch_spread_w(const SpreadJob<R> *jobs, const int *tile0s, int njobs, con
             hipLaunchKernelGGL((k_spread_narrow<W, false>), dim3((unsigned)persistent_grid(fn, NarrowCfg::NT, lds)),
                                dim3(NarrowCfg::NT), lds, st, jobs, tile0s, njobs, xr, wc, fbl);
         }
-        // the tiles the narrow kernel queued (usually none: its workgroups then
+        // those the narrow kernel queued (usually none: the workgroups then
         // only read the empty count)
-        hipLaunchKernelGGL((k_spread_wide<R, W>), dim3((unsigned)persistent_grid(fw, NT, lds)), dim3(NT), lds, st,
-                           jobs, tile0s, njobs, xr, wc, (const int *)fbl);
+        items = fbl;
+    }
+    if (real) {
+        const void *fw = reinterpret_cast<const void *>(&k_spread_wide<R, W, true>);
+        hipLaunchKernelGGL((k_spread_wide<R, W, true>), dim3((unsigned)persistent_grid(fw, NT, lds)), dim3(NT), lds, st,
+                           jobs, tile0s, njobs, xr, wc, items);
     } else {
-        hipLaunchKernelGGL((k_spread_wide<R, W>), dim3((unsigned)persistent_grid(fw, NT, lds)), dim3(NT), lds, st,
-                           jobs, tile0s, njobs, xr, wc, (const int *)nullptr);
+        const void *fw = reinterpret_cast<const void *>(&k_spread_wide<R, W, false>);
+        hipLaunchKernelGGL((k_spread_wide<R, W, false>), dim3((unsigned)persistent_grid(fw, NT, lds)), dim3(NT), lds,
+                           st, jobs, tile0s, njobs, xr, wc, items);
     }
 }
 
 #define MPSQ_SPREAD_W_ARGS(R)                                                                                         \
-    const SpreadJob<R> *, const int *, int, const int *, int *, int *, size_t, hipStream_t, size_t
+    const SpreadJob<R> *, const int *, int, const int *, int *, int *, size_t, hipStream_t, bool, size_t
 // declared here, instantiated in one spread_w*.hip each
 #define MPSQ_SPREAD_W_EXTERN(W)                                                                                       \
     extern template void launch_spread_w<float, W>(MPSQ_SPREAD_W_ARGS(float));                                        \

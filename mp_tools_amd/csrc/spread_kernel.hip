@@ -26,18 +26,18 @@ size_t spread_lds_real(int rows, int n1, int w)
 {
     return (size_t)spread_real_tw_offset(rows, n1, w) + (size_t)n1 * 8 + (size_t)(n1 / 2) * 4 + (size_t)rows * 8;
 }
-bool spread_real_ok(int rows, int, int) { return spread_real_fits(rows); }
+template <typename R> bool spread_real_ok(int rows) { return sizeof(R) == 8 || spread_real_fits(rows); }
 template <typename R> int spread_tile_elems() { return SpreadCfg<R>::E * SpreadCfg<R>::NT; }
 int spread_max_runs() { return MAX_RUNS; }
 int spread_max_tile_b() { return MAX_TILE_B; }
 int spread_max_wide_passes() { return MAX_WIDE_PASSES; }
-template <typename R> size_t spread_lds(int rows, int n1, int w, bool real)
+template <typename R> size_t spread_lds(int by, int bz, int n1, int w, bool real)
 {
-    return spread_lds_bytes<R>(rows, n1, w, real);
+    return spread_lds_bytes<R>(by, bz, n1, w, real);
 }
-template <typename R> size_t spread_lds_twiddles(int rows, int n1, int w, bool real)
+template <typename R> size_t spread_lds_twiddles(int by, int bz, int n1, int w, bool real)
 {
-    return spread_tile_bytes<R>(rows, n1, w, real);
+    return spread_tile_bytes<R>(by, bz, n1, w, real);
 }
 
 __global__ void k_zero_i32(int *__restrict__ p, int n)
@@ -53,11 +53,11 @@ void launch_zero_i32(int *p, int n, hipStream_t st)
 
 template <typename R>
 void launch_spread_jobs(const SpreadJob<R> *jobs, const int *tile0s, int njobs, int w, const int *xr, int *wc,
-                        int *fbl, size_t lds, hipStream_t st, size_t lds_real)
+                        int *fbl, size_t lds, hipStream_t st, bool real, size_t lds_real)
 {
     if (njobs <= 0) return;
 #define MPSQ_SPREAD_W(WV)                                                                                             \
-    case WV: launch_spread_w<R, WV>(jobs, tile0s, njobs, xr, wc, fbl, lds, st, lds_real); break;
+    case WV: launch_spread_w<R, WV>(jobs, tile0s, njobs, xr, wc, fbl, lds, st, real, lds_real); break;
     switch (w) {
         MPSQ_SPREAD_W(2)
         MPSQ_SPREAD_W(3)
@@ -80,13 +80,14 @@ void launch_spread_jobs(const SpreadJob<R> *jobs, const int *tile0s, int njobs, 
 }
 
 #define MPSQ_SPREAD_INST(R)                                                                                           \
+    template bool spread_real_ok<R>(int);                                                                             \
     template int spread_tile_elems<R>();                                                                              \
     template int spread_max_rows<R>(int);                                                                             \
-    template int spread_group_rows<R>(int, int);                                                                      \
-    template size_t spread_lds<R>(int, int, int, bool);                                                               \
-    template size_t spread_lds_twiddles<R>(int, int, int, bool);                                                      \
+    template int spread_group_rows<R>(int, int, int, bool);                                                           \
+    template size_t spread_lds<R>(int, int, int, int, bool);                                                          \
+    template size_t spread_lds_twiddles<R>(int, int, int, int, bool);                                                 \
     template void launch_spread_jobs<R>(const SpreadJob<R> *, const int *, int, int, const int *, int *, int *,      \
-                                        size_t, hipStream_t, size_t);
+                                        size_t, hipStream_t, bool, size_t);
 
 MPSQ_SPREAD_INST(float)
 MPSQ_SPREAD_INST(double)

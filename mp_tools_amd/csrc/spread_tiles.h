@@ -27,10 +27,12 @@ __host__ __device__ inline int posmod(int a, int n)
     return r < 0 ? r + n : r;
 }
 
-// sort bins a tile visits: y bins [ylo, ylo + nyb), z bins [zlo, zlo + nzb) (cyclic)
-__host__ __device__ inline void tile_bins(const Geo &g, int y0, int z0, int &ylo, int &nyb, int &zlo, int &nzb)
+// sort bins that by x bz rows from (y0, z0) visit: y bins [ylo, ylo + nyb),
+// z bins [zlo, zlo + nzb) (cyclic)
+__host__ __device__ inline void rect_bins(const Geo &g, int y0, int z0, int by, int bz, int &ylo, int &nyb, int &zlo,
+                                          int &nzb)
 {
-    const int w = g.w, by = (g.dim >= 2) ? g.by : 1, bz = (g.dim >= 3) ? g.bz : 1;
+    const int w = g.w;
     ylo = 0;
     nyb = 1;
     zlo = 0;
@@ -51,6 +53,12 @@ __host__ __device__ inline void tile_bins(const Geo &g, int y0, int z0, int &ylo
             nzb = g.nbZ;
         }
     }
+}
+
+// the same for a whole tile
+__host__ __device__ inline void tile_bins(const Geo &g, int y0, int z0, int &ylo, int &nyb, int &zlo, int &nzb)
+{
+    rect_bins(g, y0, z0, (g.dim >= 2) ? g.by : 1, (g.dim >= 3) ? g.bz : 1, ylo, nyb, zlo, nzb);
 }
 
 // runs of a tile: 2 per visited z-bin row (the second one is empty unless

@@ -118,3 +118,39 @@ def test_real_long_rows(gpu_lib, precision, eps, tol):
     torch.cuda.synchronize()
     F = _oracle(pos, counts, nm, ncell, False)
     assert rel_l2(amp.cpu().numpy(), (F * w[None, :, None]).sum(axis=1)) < tol
+
+
+# tiles whose rows do not split into equal powers of two: one pass of an odd
+# number of rows (the last FFT pair lacks its second row), passes that are
+# parts of one plane, single rows, a whole small grid
+@pytest.mark.parametrize("precision,eps,tol", [("fp32", 1e-6, 2e-5), ("fp64", 1e-10, 1e-8)])
+@pytest.mark.parametrize("q0", [0.0, 0.25])
+@pytest.mark.parametrize("nm,by,bz", [((64, 24, 10), 3, 5), ((64, 24, 10), 1, 1), ((64, 24, 10), 6, 1), ((400, 24, 10), 6, 1),
+                                      ((500, 24, 10), 2, 2), ((64, 24, 10), 4, 4), ((700, 24), 3, 0), ((300, 24), 8, 0)])
+def test_wide_pass_shapes(gpu_lib, precision, eps, tol, q0, nm, by, bz):
+    import torch
+    from mp_tools_amd.sqw import SqwEngine
+    rng = np.random.default_rng(by * 10 + bz)
+    ncell, T, n = 4, 2, 9000
+    counts = np.array([n // 2, n // 2])
+    pos = np.zeros((T, n, 4), np.float32)
+    pos[:, :, :3] = rng.uniform(0.0, ncell, (T, n, 3))
+    pos[:, ::3, 1:3] = 1.25 + 0.001 * pos[:, ::3, 1:3]  # a third of the points in few rows: dense tiles
+    w = np.array([0.6, -0.4])
+    kw = dict(eps=eps, precision=precision, weights=w, tpe=(2 * np.pi / ncell,) * 3, q0=(q0, 0.0, 0.0), tile_by=by,
+              tile_bz=bz)
+    if precision == "fp64" and q0 and by * max(bz, 1) * 2 * nm[0] > 4096:  # more rows than its pass takes
+        from mp_tools_amd._lib import MpsqError
+        with pytest.raises(MpsqError):
+            SqwEngine(len(nm), nm, counts, **kw)
+        return
+    eng = SqwEngine(len(nm), nm, counts, **kw)
+    amp = eng.amplitudes(torch.tensor(pos, device="cuda")).cpu().numpy()
+    off = [0, n // 2, n]
+    for t in range(T):
+        f = 0.0
+        for j in range(2):
+            x, y, z, c = O.stage(pos[t, off[j]:off[j + 1]], None, (0, 0, 0), np.eye(3), (2 * np.pi / ncell,) * 3,
+                                 (q0, 0.0, 0.0), False, 1.0, dim=len(nm))
+            f = f + w[j] * O.dirft_type1(x, y, z if len(nm) == 3 else None, c, nm).ravel()
+        assert rel_l2(amp[t], f) < tol
