@@ -295,6 +295,15 @@ int mpsq_sqw_debug_sorted(mpsq_sqw eng, const float *d_pos, int64_t frame, int32
 /* Fine grid, kernel width, spread tile and sort-bin shape of an engine, in
  * the layout of mpsq_plan_info. */
 int mpsq_sqw_info(mpsq_sqw eng, int64_t *out);
+/* Bytes of the intermediate grids of a run of `frames` frames, and their
+ * placement in the caller's device memory (256-byte aligned) instead of
+ * memory that the engine allocates: for a program that makes engines of
+ * large grids again and again and keeps the memory itself.  The memory must
+ * not be freed or used otherwise while the engine runs; d_ws = NULL ends the
+ * loan (the engine then allocates again).  Runs of more frames than `frames`
+ * allocate. */
+int64_t mpsq_sqw_workspace(mpsq_sqw eng, int64_t frames);
+int mpsq_sqw_set_workspace(mpsq_sqw eng, void *d_ws, int64_t bytes, int64_t frames);
 /* Synchronise the engine's stream. */
 int mpsq_sqw_sync(mpsq_sqw eng);
 /* Per-stage timing with HIP events recorded on the engine's stream around

@@ -36,6 +36,7 @@ EXPORTS = [
     "mpsq_sqw_default_spec", "mpsq_sqw_create", "mpsq_sqw_amplitudes", "mpsq_sqw_reduce",
     "mpsq_sqw_destroy", "mpsq_sqw_sync", "mpsq_sqw_nq", "mpsq_sqw_nact", "mpsq_version",
     "mpsq_sqw_set_timing", "mpsq_sqw_get_timing", "mpsq_sqw_debug_sorted", "mpsq_sqw_info", "mpsq_qtables",
+    "mpsq_sqw_workspace", "mpsq_sqw_set_workspace",
     "mpsq_speckle_filter", "mpsq_oneph_amplitudes", "mpsq_dos",
     "mpsq_batch_create", "mpsq_batch_run", "mpsq_batch_set_budget", "mpsq_batch_set_timing",
     "mpsq_batch_get_timing", "mpsq_batch_destroy", "mpsq_autotune_tiles",
@@ -163,6 +164,9 @@ def load():
     L.mpsq_oneph_amplitudes.argtypes = [vp, vp, vp, i64, vp, vp, vp, vp]
     L.mpsq_dos.argtypes = [vp, i64, i64, vp, i32, i64, i32, vp, vp]
     L.mpsq_sqw_info.argtypes = [vp, vp]
+    L.mpsq_sqw_workspace.argtypes = [vp, i64]
+    L.mpsq_sqw_workspace.restype = i64
+    L.mpsq_sqw_set_workspace.argtypes = [vp, vp, i64, i64]
     L.mpsq_sqw_get_timing.argtypes = [vp, vp, vp, i32]
     L.mpsq_batch_create.argtypes = [i32, vp, vp]
     L.mpsq_batch_run.argtypes = [vp, vp, vp, vp, vp, vp, vp, i32]

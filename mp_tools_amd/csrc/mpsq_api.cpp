@@ -45,6 +45,15 @@ static void throw_bad(int hbad)
 struct DevBuf {
     void *p = nullptr;
     size_t bytes = 0;
+    bool lent = false;  // the memory is the caller's
+    // use the caller's memory (which outlives the buffer's use of it)
+    void adopt(void *q, size_t b)
+    {
+        release();
+        p = q;
+        bytes = b;
+        lent = true;
+    }
     void ensure(size_t b)
     {
         if (b <= bytes && p) return;
@@ -58,9 +67,10 @@ struct DevBuf {
     }
     void release()
     {
-        if (p) (void)hipFree(p);
+        if (p && !lent) (void)hipFree(p);
         p = nullptr;
         bytes = 0;
+        lent = false;
     }
     template <typename T> T *as() const { return static_cast<T *>(p); }
     ~DevBuf() { release(); }
@@ -1136,6 +1146,36 @@ template <typename R> struct Engine {
         int b = s->batch_frames > 0 ? std::min(s->batch_frames, 1024)
                                     : (int)std::min<size_t>(std::max<size_t>(1, budget / bytes_per_frame(tpf)), 128);
         B = std::max(1, b);
+    }
+
+    // bytes of the two intermediate grids of a run of `frames` frames, each
+    // rounded up to 256 (the column passes' half spectrum as run_parts lays
+    // it out)
+    void grid_bytes(int64_t frames, size_t &g1, size_t &g2) const
+    {
+        const Core<R> &c = core;
+        const bool herm = c.real_launch() && !(combine && wtab.p);
+        const size_t ntr = (size_t)std::min<int64_t>(frames, B) * (size_t)((combine && !wtab.p) ? 1 : nact);
+        const size_t row = sizeof(Cx<R>) * ntr * (size_t)(c.n[2] * c.h1x(herm));
+        auto up = [](size_t b) { return (b + 255) / 256 * 256; };
+        g1 = up(row * (size_t)c.n[1]);
+        g2 = c.dim == 3 ? up(row * (size_t)(herm ? c.N[1] + 1 : c.N[1])) : 0;
+    }
+    // the intermediate grids in the caller's memory
+    void set_workspace(void *ptr, size_t bytes, int64_t frames)
+    {
+        size_t g1, g2;
+        grid_bytes(frames, g1, g2);
+        HIPCHK(hipSetDevice(core.device));
+        HIPCHK(hipStreamSynchronize(core.st));  // no run still uses the present grids
+        if (!ptr) {
+            ws.G1.release();
+            ws.G2.release();
+            return;
+        }
+        if (bytes < g1 + g2 || (uintptr_t)ptr % 256) throw Err{MPSQ_ERR_BAD_ARG};
+        ws.G1.adopt(ptr, g1);
+        if (g2) ws.G2.adopt(static_cast<unsigned char *>(ptr) + g1, g2);
     }
 
     void amplitudes(const float *d_pos, int64_t T, void *d_amp)
@@ -2615,6 +2655,29 @@ int mpsq_sqw_info(mpsq_sqw e, int64_t *out)
     const Geo &g = e->ed ? e->ed->core.g : e->ef->core.g;
     const int64_t v[8] = {g.n1, g.n2, g.n3, g.w, g.by, g.bz, g.BY, g.BZ};
     for (int k = 0; k < 8; ++k) out[k] = v[k];
+    return 0;
+}
+
+int64_t mpsq_sqw_workspace(mpsq_sqw e, int64_t frames)
+{
+    if (!e || frames < 1) return 0;
+    size_t g1, g2;
+    if (e->ed) e->ed->grid_bytes(frames, g1, g2);
+    else e->ef->grid_bytes(frames, g1, g2);
+    return (int64_t)(g1 + g2);
+}
+
+int mpsq_sqw_set_workspace(mpsq_sqw e, void *d_ws, int64_t bytes, int64_t frames)
+{
+    if (!e || frames < 1 || bytes < 0) return MPSQ_ERR_BAD_ARG;
+    try {
+        if (e->ed) e->ed->set_workspace(d_ws, (size_t)bytes, frames);
+        else e->ef->set_workspace(d_ws, (size_t)bytes, frames);
+    } catch (const Err &er) {
+        return er.code;
+    } catch (...) {
+        return MPSQ_ERR_DEVICE;
+    }
     return 0;
 }
 

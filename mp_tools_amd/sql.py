@@ -114,7 +114,7 @@ def histogram(frames, counts, geo: SqlGeometry, eps: float = 1e-6, precision: st
     if mc and n_mc == N_MC and n_h > n_h_max(geo):
         raise ValueError(f"n_h exceeds the {n_h_max(geo)} chains of 10^6 samples this Q box allows (mp_sql56.f90:1069)")
 
-    from .nufft import Plan
+    from .sqw import SqwEngine
     L = _lib.load()
     nsp = len(counts)
     npairs = nsp * (nsp + 1) // 2
@@ -127,7 +127,13 @@ def histogram(frames, counts, geo: SqlGeometry, eps: float = 1e-6, precision: st
     amp = torch.empty((nsp, nq), dtype=cdt, device=dev)
     off = np.concatenate([[0], np.cumsum(counts)])
     stream = torch.cuda.current_stream(dev)
-    plans = [Plan(1, geo.n_qq, eps=eps, isign=-1, dtype=dtype, device=device, stream="torch") for _ in range(nsp)]
+    # One engine per species: amplitudes of unit strengths in the species'
+    # REAL(4) coordinates x = at_pos * d_q (mp_sql56.f90:1115-1118).  The
+    # strengths are real, so the engine spreads real cells and transforms half
+    # the spectrum; its grids share one torch buffer, which torch's allocator
+    # keeps between calls (allocated and freed in every call, the grids of
+    # 509^3 modes cost 650 ms of a 720 ms call).
+    engines, buf = [None] * nsp, None
     ev0, ev1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
     ev0.record(stream)
     skip = torch.zeros(2, dtype=torch.int64, device=dev)
@@ -137,13 +143,18 @@ def histogram(frames, counts, geo: SqlGeometry, eps: float = 1e-6, precision: st
         pos = np.asarray(pos)
         for s in range(nsp):
             r = pos[off[s]:off[s + 1], :3].astype(np.float32)
-            # x = at_pos * d_q in FP32 (mp_sql56.f90:1115-1118), handed on as FP64
-            xyz = [torch.tensor((r[:, d] * geo.dq[d]).astype(np.float64), device=dev) for d in range(3)]
-            if precision != "fp64":
-                xyz = [v.float() for v in xyz]
-            plans[s].setpts(*xyz)
-            c = torch.ones(len(r), dtype=cdt, device=dev)
-            amp[s] = plans[s].execute(c).reshape(-1)
+            if len(r) == 0:
+                amp[s].zero_()
+                continue
+            x = torch.zeros((1, len(r), 4), dtype=torch.float32, device=dev)
+            x[0, :, :3] = torch.from_numpy(r * geo.dq).to(dev)
+            if engines[s] is None or engines[s].n_tot != len(r):
+                engines[s] = SqwEngine(3, geo.n_qq, (len(r),), eps=eps, precision=precision, combine=False, tpe=(1.0,) * 3,
+                                       vacancy_check=False, device=device, stream=stream.cuda_stream)
+                if buf is None or buf.numel() < engines[s].workspace_bytes():
+                    buf = torch.empty(engines[s].workspace_bytes(), dtype=torch.uint8, device=dev)
+                engines[s].set_workspace(buf)
+            engines[s].amplitudes(x, out=amp[s])
         nm = (C.c_int64 * 3)(N1, N2, N3)
         dq = (C.c_float * 3)(*[float(v) for v in geo.dq])
         ai = (C.c_float * 9)(*[float(v) for v in geo.a_cell_inv.reshape(-1)])

@@ -199,6 +199,19 @@ class SqwEngine:
         _lib.check("sqw_debug_sorted", rc)
         return atom, cell, keep
 
+    def workspace_bytes(self, frames=1):
+        """Bytes of the intermediate grids of a run of ``frames`` frames."""
+        return int(self._L.mpsq_sqw_workspace(self._h, int(frames)))
+
+    def set_workspace(self, buf, frames=1):
+        """Keep the intermediate grids of runs of up to ``frames`` frames in
+        the CUDA tensor ``buf`` (held until another is set; None: memory of
+        the engine's own)."""
+        n = 0 if buf is None else buf.numel() * buf.element_size()
+        _lib.check("sqw_set_workspace", self._L.mpsq_sqw_set_workspace(self._h, None if buf is None else buf.data_ptr(),
+                                                                      n, int(frames)))
+        self._ws = buf
+
     def info(self):
         """Fine grid, kernel width, spread tile and sort-bin shape."""
         out = (C.c_int64 * 8)()
