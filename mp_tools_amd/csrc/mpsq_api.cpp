@@ -450,7 +450,7 @@ template <typename R> struct Core {
         es_params(eps, sizeof(R) == 4, w, beta, warn);
         for (int d = 0; d < 3; ++d) n[d] = (d < dim) ? next_smooth_even(std::max(2 * N[d], (int64_t)2 * w)) : 1;
         const int TE = spread_tile_elems<R>();
-        const int TC = colfft_tile_elems<R>(true);
+        const int TC = colfft_max_len<R>();
         if (n[0] > TE || n[1] > TC || n[2] > TC) throw Err{MPSQ_ERR_SIZE};
         g.dim = dim;
         g.n1 = (int)n[0];
@@ -477,14 +477,20 @@ template <typename R> struct Core {
         // re-walks the whole tile's candidates
         rows_max = spread_max_rows<R>((int)n[0]);
         if (real && rows_max < 32) rows_max = std::min(2 * rows_max, 32);
+        // FP64 tiles of real strengths: no more rows than let two workgroups
+        // share a CU (fine rows of 1024 cells: 4 rows, 51 KB, instead of 8,
+        // 86 KB; 30,000 points 0.124 -> 0.113 ms, 3 million 1.62 -> 1.49)
+        int rows_def = rows_max;
+        while (real && sizeof(R) == 8 && rows_def > 2 && spread_lds<R>(rows_def, 1, (int)n[0], w, true) > 80 * 1024)
+            rows_def /= 2;
         const int bmax = spread_max_tile_b();
         int by = 1, bz = 1;
         if (dim == 2) {
-            for (int b = 1; b <= rows_max && b <= bmax && n[1] % b == 0 && b + w <= n[1]; b *= 2) by = b;
+            for (int b = 1; b <= rows_def && b <= bmax && n[1] % b == 0 && b + w <= n[1]; b *= 2) by = b;
         } else if (dim == 3) {
             double best = 1e300;
-            for (int b1 = 1; b1 <= rows_max && b1 <= bmax && n[1] % b1 == 0 && b1 + w <= n[1]; b1 *= 2)
-                for (int b2 = 1; b1 * b2 <= rows_max && b2 <= bmax && n[2] % b2 == 0 && b2 + w <= n[2]; b2 *= 2) {
+            for (int b1 = 1; b1 <= rows_def && b1 <= bmax && n[1] % b1 == 0 && b1 + w <= n[1]; b1 *= 2)
+                for (int b2 = 1; b1 * b2 <= rows_def && b2 <= bmax && n[2] % b2 == 0 && b2 + w <= n[2]; b2 *= 2) {
                     // (ties: more rows, then the taller y extent, whose
                     // covering bounds, summed over fewer z-bin rows, are
                     // smaller: C2's real 8 x 4 tiles give 1.51e-5 at random
@@ -557,16 +563,6 @@ template <typename R> struct Core {
 
     int keybits() const { return g.nbins > 1 ? ilog2_ceil(g.nbins) : 0; }
 
-    int colfft_cols(int64_t nlen, int64_t inner, bool final) const
-    {
-        const int TE = (final && nlen <= colfft_final_small_elems<R>()) ? colfft_final_small_elems<R>()
-                                                                         : colfft_tile_elems<R>(final);
-        int c = 1;
-        while ((int64_t)(2 * c) * nlen <= TE) c *= 2;
-        while (c > 1 && c / 2 >= inner) c /= 2;
-        return c;
-    }
-
     // Column passes after spreading.  2D: one final pass along y.  3D: a
     // y pass (every transform) and a final z pass that groups nsp
     // consecutive transforms (species) with their weights.  herm (real
@@ -577,7 +573,7 @@ template <typename R> struct Core {
     // segments of the y pass start on cache lines)
     int64_t h1v(bool herm) const { return herm ? N[0] / 2 + 1 : N[0]; }
     int64_t h1x(bool herm) const { return herm ? (h1v(true) + 15) / 16 * 16 : N[0]; }
-    ColPass colpass(int axis, bool final, int nsp, bool herm = false) const
+    ColPass colpass(int axis, bool final, int nsp, int ngroups, bool herm = false) const
     {
         ColPass c{};
         const int64_t NQ = N[0] * N[1] * N[2];
@@ -606,7 +602,7 @@ template <typename R> struct Core {
             c.hsa = (dim == 3) ? N[0] * N[1] : N[0];
             c.dH1 = make_fdiv((uint32_t)H1);
         }
-        c.cols = colfft_cols(c.n, c.inner, final);
+        c.cols = colfft_cols<R>(c.n, c.inner, (int64_t)c.outer * ngroups, final);
         c.dcols = make_fdiv((uint32_t)c.cols);
         c.nsp = nsp;
         c.NQ = NQ;
@@ -617,7 +613,7 @@ template <typename R> struct Core {
                      const float *wtab, bool herm = false) const
     {
         ColJob<R> J{};
-        J.cp = colpass(axis, final, nsp, herm);
+        J.cp = colpass(axis, final, nsp, ngroups, herm);
         J.rp = rp[axis];
         J.in = in;
         J.out = out;
@@ -866,11 +862,11 @@ template <typename R> struct Plan {
         if (!cy.empty())
             launch_colfft_jobs<R>(run_tab.dev<ColJob<R>>(o_cy), run_tab.dev<int>(o_z), 1,
                                   (int)Core<R>::col_blocks(cy[0]), false, colfft_lds<R>(cy[0].cp, false), c.st,
-                                  cy[0].cp.n);
+                                  cy[0].cp.n * cy[0].cp.cols, cy[0].cp.cols);
         if (!cz.empty())
             launch_colfft_jobs<R>(run_tab.dev<ColJob<R>>(o_cz), run_tab.dev<int>(o_z), 1,
                                   (int)Core<R>::col_blocks(cz[0]), true, colfft_lds<R>(cz[0].cp, true), c.st,
-                                  cz[0].cp.n);
+                                  cz[0].cp.n * cz[0].cp.cols, cz[0].cp.cols);
         HIPCHK(hipGetLastError());
         if (!on_device) {
             int hbad = 0;
@@ -1629,15 +1625,21 @@ static void run_parts(const std::vector<Part<R>> &parts, Workspace<R> &ws, Arena
         launch_spread_jobs<R>(A.dev<SpreadJob<R>>(L.o_jobs), A.dev<int>(L.o_t0), L.njobs, L.w, A.dev<int>(L.o_xr),
                               ws.wc.template as<int>(), ws.fbl.template as<int>(), L.lds, st, L.real, L.lds_real);
     tm->end(ev, st);
+    auto cols_of = [](const std::vector<ColJob<R>> &v) {
+        int c = 1 << 20;
+        for (const ColJob<R> &j : v) c = std::min(c, j.cp.cols);
+        return c;
+    };
     if (cyn > 0) {
         ev = tm->begin(ST_COLPASS, st);
-        launch_colfft_jobs<R>(A.dev<ColJob<R>>(o_cy), A.dev<int>(o_cyb), (int)cyj.size(), cyn, false, cyl, st, 0);
+        launch_colfft_jobs<R>(A.dev<ColJob<R>>(o_cy), A.dev<int>(o_cyb), (int)cyj.size(), cyn, false, cyl, st, 0, cols_of(cyj));
         tm->end(ev, st);
     }
     ev = tm->begin(ST_FINAL, st);
     int czmax = 0;
-    for (const ColJob<R> &cj : czj) czmax = std::max(czmax, cj.cp.n);
-    launch_colfft_jobs<R>(A.dev<ColJob<R>>(o_cz), A.dev<int>(o_czb), (int)czj.size(), czn, true, czl, st, czmax);
+    for (const ColJob<R> &cj : czj) czmax = std::max(czmax, cj.cp.n * cj.cp.cols);
+    launch_colfft_jobs<R>(A.dev<ColJob<R>>(o_cz), A.dev<int>(o_czb), (int)czj.size(), czn, true, czl, st, czmax,
+                          cols_of(czj));
     tm->end(ev, st);
 }
 

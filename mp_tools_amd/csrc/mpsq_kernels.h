@@ -219,10 +219,10 @@ size_t spread_lds_real(int rows, int n1, int w);
 template <typename R>
 void launch_binmax(const PtRec<R> *srec, const int64_t *binstart, const TransformInfo *tinfo, int ntr, int max_nbins,
                    int *binmax, hipStream_t st);
-template <typename R> int colfft_tile_elems(bool final);
-// columns of length n <= colfft_final_small_elems() take the final pass's
-// smaller tile (and its blocks of fewer threads)
-template <typename R> int colfft_final_small_elems();
+// longest column of the column passes, and the columns one workgroup takes
+// (columns of n rows, `inner` adjacent ones in each of `slabs` slabs)
+template <typename R> int colfft_max_len();
+template <typename R> int colfft_cols(int64_t n, int64_t inner, int64_t slabs, bool final);
 // Spread + x FFT of every tile of a job table in one persistent launch.
 // Workgroups run on XCD blockIdx.x % 8 and take tiles of their XCD's range
 // [xr[x], xr[x+1]) of the tile-id space from the counter
@@ -271,9 +271,11 @@ void launch_zero_i32(int *p, int n, hipStream_t st);
 // amax[t] = max over the M strengths of transform t of max(|Re|, |Im|)
 void launch_absmax(int64_t M, int ntr, const float2 *c, float *amax, hipStream_t st);
 template <typename R> size_t colfft_lds(const ColPass &cp, bool final);
+// (max_elems: the jobs' largest cols * n; min_cols: their fewest columns per
+// workgroup)
 template <typename R>
 void launch_colfft_jobs(const ColJob<R> *jobs, const int *blk0s, int njobs, int nblocks, bool final, size_t lds,
-                        hipStream_t st, int max_n);
+                        hipStream_t st, int max_elems, int min_cols);
 
 // --- launch helpers (sqw_kernels.hip) ---
 // X-ray form-factor weights w[s][Q] on the mode grid N (see sqw_kernels.hip)

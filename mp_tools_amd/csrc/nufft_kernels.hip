@@ -475,25 +475,38 @@ __global__ void k_absmax(int64_t M, const float2 *__restrict__ c, unsigned *__re
 // RC is the arithmetic (and LDS tile) precision; the data in HBM stays
 // cplx<R> (RC = double on FP32 data runs the pass in FP64 with FP64
 // twiddles).
+// Work block of a launched one where neighbouring column blocks share
+// 128-byte lines (row segments below that: FP64 columns of 1024 rows have 64
+// bytes): workgroups go to the 8 XCDs in turn, and each XCD takes one
+// contiguous range of the blocks, so that a line is fetched into one L2 only.
+// (y pass of 1024-row FP64 columns 1.9 -> 1.6 ms; with whole-line segments
+// the order makes no difference, or costs up to half a percent.)
+__device__ __forceinline__ int xcd_block(int b, int nb)
+{
+    const int x = b & 7, q = nb >> 3, r = nb & 7;
+    return x * q + min(x, r) + (b >> 3);
+}
+
 template <typename R, typename RC, int E, int NT, bool FINAL>
 __global__ __launch_bounds__(NT) void k_colfft(const ColJob<R> *__restrict__ jobs, const int *__restrict__ blk0s,
-                                               int njobs)
+                                               int njobs, int by_xcd)
 {
     using C = typename cplx<RC>::T;
     using CS = typename cplx<R>::T;
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    const ColJob<R> &J = jobs[find_job(blk0s, njobs, blockIdx.x)];
+    const int blk = by_xcd ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
+    const ColJob<R> &J = jobs[find_job(blk0s, njobs, blk)];
     const ColPass &cp = J.cp;
     C *tile = reinterpret_cast<C *>(smem_raw);
     const int n = cp.n, N = cp.N, cols = cp.cols, inner = cp.inner;
     C *tw_l = tile + n * cols;  // twiddles in LDS
-    C *acc = tw_l + n;          // FINAL: species sum of the kept modes, [NO][cols]
+    C *acc = tw_l + n;          // FINAL, nsp > 1: species sum of the kept modes, [NO][cols]
     const C *twg;
     if constexpr (sizeof(RC) == sizeof(R)) twg = reinterpret_cast<const C *>(J.tw);
     else twg = reinterpret_cast<const C *>(J.tw64);
     for (int i = threadIdx.x; i < n; i += NT) tw_l[i] = twg[i];
     const int ncb = J.ncb;
-    const int local = blockIdx.x - J.blk0;
+    const int local = blk - J.blk0;
     const int grp = local / (ncb * cp.outer);
     const int rem = local - grp * ncb * cp.outer;
     const int o = rem / ncb, cb = rem - o * ncb;
@@ -505,6 +518,31 @@ __global__ __launch_bounds__(NT) void k_colfft(const ColJob<R> *__restrict__ job
     // extra half-spectrum output k = N - h takes that of -k (entry 0 for
     // even N; for odd N that output is never a mirror source)
     auto phi_ix = [&](int kk) { return kk < N ? kk : 0; };
+    // FINAL: output kk of column c to the map.  herm: column col = km * hH1 +
+    // kh (3D; 2D: col = kh); the transformed axis' index kk.  Mode (kk, km,
+    // kh) goes to its place and, when k1 < 0, its mirror (2 h - kk, 2 h2 - km,
+    // 2 h1 - kh), where in range, as the conjugate: every mode of the map is
+    // written once.
+    auto emit = [&](int kk, int c, CS x) {
+        if (cp.conj) x.y = -x.y;
+        CS *dst = J.out + (int64_t)grp * cp.out_tstride;
+        if (!cp.herm) {
+            if (kk < N) dst[(int64_t)o * N * inner + col0 + (int64_t)kk * inner + c] = x;
+            return;
+        }
+        const int N1 = cp.hN1, h1 = N1 / 2, N2 = cp.hN2, h2 = N2 / 2;
+        const int col = col0 + c;
+        int km = 0, kh = col;
+        if (cp.hmid) {
+            km = (int)fdiv((uint32_t)col, cp.dH1);
+            kh = col - km * cp.hH1;
+        }
+        if (kh >= cp.hH1v) return;  // pad column
+        if (kk < N && km < N2) dst[(int64_t)kk * cp.hsa + (int64_t)km * N1 + kh] = x;
+        const int ka = 2 * h - kk, kmm = cp.hmid ? 2 * h2 - km : 0, kx = 2 * h1 - kh;
+        if (kh < h1 && kx < N1 && ka >= 0 && ka < N && kmm >= 0 && kmm < N2)
+            dst[(int64_t)ka * cp.hsa + (int64_t)kmm * N1 + kx] = cmk<CS>(x.x, -x.y);
+    };
     for (int s = 0; s < nsp; ++s) {
         const int t = FINAL ? grp * cp.nsp + s : grp;
         {
@@ -554,47 +592,13 @@ __global__ __launch_bounds__(NT) void k_colfft(const ColJob<R> *__restrict__ job
                 // (a half-spectrum pass has no per-Q table: the host keeps those jobs full)
                 if (J.wtab) wv *= (c < ncol) ? (R)J.wtab[(int64_t)s * cp.NQ + (int64_t)kk * inner + col0 + c] : (R)0;
                 else if (J.wsc) wv *= J.wsc[s];
-                const C x = cscale(tile[f * cols + c], wv);
-                acc[i] = (s == 0) ? x : cadd(acc[i], x);
+                C x = cscale(tile[f * cols + c], wv);
+                if (s > 0) x = cadd(acc[i], x);
+                if (s + 1 < nsp) acc[i] = x;
+                else if (c < ncol) emit(kk, c, x);
             }
         }
         __syncthreads();
-    }
-    if constexpr (FINAL) {
-        if (!cp.herm) {
-            C *dst = J.out + (int64_t)grp * cp.out_tstride + (int64_t)o * N * inner + col0;
-            for (int i = threadIdx.x; i < N * cols; i += NT) {
-                const int kk = (int)fdiv((uint32_t)i, cp.dcols), c = i - kk * cols;
-                if (c >= ncol) continue;
-                C x = acc[i];
-                if (cp.conj) x.y = -x.y;
-                dst[(int64_t)kk * inner + c] = x;
-            }
-        } else {
-            // column col = km * hH1 + kh (3D; 2D: col = kh); the transformed
-            // axis' index kk.  Mode (kk, km, kh) goes to its place and, when
-            // k1 < 0, its mirror (2 h - kk, 2 h2 - km, 2 h1 - kh), where in
-            // range, as the conjugate: every mode of the map is written once.
-            C *dst = J.out + (int64_t)grp * cp.out_tstride;
-            const int N1 = cp.hN1, h1 = N1 / 2, N2 = cp.hN2, h2 = N2 / 2;
-            for (int i = threadIdx.x; i < NO * cols; i += NT) {
-                const int kk = (int)fdiv((uint32_t)i, cp.dcols), c = i - kk * cols;
-                if (c >= ncol) continue;
-                const int col = col0 + c;
-                int km = 0, kh = col;
-                if (cp.hmid) {
-                    km = (int)fdiv((uint32_t)col, cp.dH1);
-                    kh = col - km * cp.hH1;
-                }
-                C x = acc[i];
-                if (cp.conj) x.y = -x.y;
-                if (kh >= cp.hH1v) continue;  // pad column
-                if (kk < N && km < N2) dst[(int64_t)kk * cp.hsa + (int64_t)km * N1 + kh] = x;
-                const int ka = 2 * h - kk, kmm = cp.hmid ? 2 * h2 - km : 0, kx = 2 * h1 - kh;
-                if (kh < h1 && kx < N1 && ka >= 0 && ka < N && kmm >= 0 && kmm < N2)
-                    dst[(int64_t)ka * cp.hsa + (int64_t)kmm * N1 + kx] = cmk<C>(x.x, -x.y);
-            }
-        }
     }
 }
 
@@ -604,12 +608,13 @@ __global__ __launch_bounds__(NT) void k_colfft(const ColJob<R> *__restrict__ job
 template <typename R> struct Tiles;
 // y pass: 1024 threads of EY elements (FP32: 16 columns of 512 rows,
 // 128-byte row segments; two workgroups, 32 waves, per CU); final pass:
-// 256 threads of EF elements when the columns fit (FP32 on C2: 32 columns of
-// 64 rows, 256-byte row segments), small tiles so that many workgroups
-// share a CU while each walks its species one after another (C2, 24
-// launches of 16 frames: 4.63 ms with 256 threads, 5.01 with 512, 4.96 with
-// 128; 4 or 16 elements per thread 5.9-6.2), else 512 threads (the size
-// limit of the column passes)
+// 256 threads of EF elements where that gives row segments of 64 bytes (FP32
+// on C2: 32 columns of 64 rows, 256-byte row segments), small tiles so that
+// many workgroups share a CU while each walks its species one after another
+// (C2, 24 launches of 16 frames: 4.63 ms with 256 threads, 5.01 with 512, 4.96
+// with 128; 4 or 16 elements per thread 5.9-6.2).  Longer columns take 512 or
+// 1024 threads while at least FINAL_BLOCKS workgroups are left: 130,560 FP64
+// columns of 1024 rows 3.85 ms with one column per workgroup, 1.88 with four.
 // RY: arithmetic of the y pass.  FP32 data keeps FP32 arithmetic: an FP64
 // y pass (8 columns of 512 rows of double2, two workgroups per CU) measured
 // 0.68 against 0.37 ms per 16-frame C2 launch, for errors of the FP32 form
@@ -617,10 +622,9 @@ template <typename R> struct Tiles;
 // of near-lattice inputs, whichever pass order)
 template <> struct Tiles<float> { static constexpr int EY = 8, EF = 8; using RY = float; };
 template <> struct Tiles<double> { static constexpr int EY = 4, EF = 4; using RY = double; };
-constexpr int colfft_nt(bool final) { return final ? 512 : 1024; }
-// the final pass in 256-thread blocks when every column of the launch fits
-constexpr int COLFFT_NT_FINAL_SMALL = 256;
-
+constexpr int COLFFT_NT_Y = 1024;
+constexpr int COLFFT_NT_FINAL[] = {256, 512, 1024};
+constexpr int64_t FINAL_BLOCKS = 1024;
 
 template <typename R>
 void launch_fold(const Geo &g, int64_t M, const void *x, const void *y, const void *z, bool in_f32, PtRec<R> *rec,
@@ -711,50 +715,71 @@ void launch_absmax(int64_t M, int ntr, const float2 *c, float *amax, hipStream_t
                        reinterpret_cast<unsigned *>(amax));
 }
 
-template <typename R> int colfft_tile_elems(bool final)
-{
-    return (final ? Tiles<R>::EF : Tiles<R>::EY) * colfft_nt(final);
-}
+// longest column (the final pass of 512 threads holds one)
+template <typename R> int colfft_max_len() { return Tiles<R>::EF * 512; }
 
-template <typename R> int colfft_final_small_elems() { return Tiles<R>::EF * COLFFT_NT_FINAL_SMALL; }
+// columns per workgroup for columns of n rows, `inner` adjacent ones in each
+// of `slabs` slabs
+template <typename R> int colfft_cols(int64_t n, int64_t inner, int64_t slabs, bool final)
+{
+    auto fit = [&](int64_t elems) {
+        int c = 1;
+        while ((int64_t)(2 * c) * n <= elems) c *= 2;
+        while (c > 1 && c / 2 >= inner) c /= 2;
+        return c;
+    };
+    if (!final) return fit((int64_t)Tiles<R>::EY * COLFFT_NT_Y);
+    int cols = 0;
+    for (int nt : COLFFT_NT_FINAL) {
+        if (n > (int64_t)Tiles<R>::EF * nt) continue;
+        const int c = fit((int64_t)Tiles<R>::EF * nt);
+        if (cols && (inner + c - 1) / c * slabs < FINAL_BLOCKS) break;
+        cols = c;
+        if (c * sizeof(typename cplx<R>::T) >= 64) break;
+    }
+    return cols;
+}
 
 // LDS of one column pass of a job: tile + twiddles (+ species sum for the final pass)
 template <typename R> size_t colfft_lds(const ColPass &cp, bool final)
 {
     const size_t es = final ? sizeof(typename cplx<R>::T) : sizeof(typename cplx<typename Tiles<R>::RY>::T);
-    return ((size_t)cp.n * (cp.cols + 1) + (final ? (size_t)cp.NO * cp.cols : 0)) * es;
+    return ((size_t)cp.n * (cp.cols + 1) + (final && cp.nsp > 1 ? (size_t)cp.NO * cp.cols : 0)) * es;
 }
 
 template <typename R>
 void launch_colfft_jobs(const ColJob<R> *jobs, const int *blk0s, int njobs, int nblocks, bool final, size_t lds,
-                        hipStream_t st, int max_n)
+                        hipStream_t st, int max_elems, int min_cols)
 {
     if (nblocks <= 0) return;
-    constexpr int EF = Tiles<R>::EF, EY = Tiles<R>::EY, NTF = colfft_nt(true), NTY = colfft_nt(false);
-    constexpr int NTS = COLFFT_NT_FINAL_SMALL;
+    constexpr int EF = Tiles<R>::EF, EY = Tiles<R>::EY, NTY = COLFFT_NT_Y;
+    constexpr int NT0 = COLFFT_NT_FINAL[0], NT1 = COLFFT_NT_FINAL[1], NT2 = COLFFT_NT_FINAL[2];
     using RY = typename Tiles<R>::RY;
     // set once per process (a function-local static initialises thread-safely)
     static const bool attr = [] {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_colfft<R, R, EF, NTF, true>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, 156 * 1024);
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_colfft<R, R, EF, NTS, true>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, 156 * 1024);
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_colfft<R, RY, EY, NTY, false>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, 156 * 1024);
+        for (const void *fn : {reinterpret_cast<const void *>(&k_colfft<R, R, EF, NT0, true>),
+                               reinterpret_cast<const void *>(&k_colfft<R, R, EF, NT1, true>),
+                               reinterpret_cast<const void *>(&k_colfft<R, R, EF, NT2, true>),
+                               reinterpret_cast<const void *>(&k_colfft<R, RY, EY, NTY, false>)})
+            (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         return true;
     }();
     (void)attr;
-    // the jobs' column counts were chosen for the small tile when their
-    // columns fit it (colfft_final_small_elems), which the large tile holds too
-    if (final && max_n <= colfft_final_small_elems<R>())
-        hipLaunchKernelGGL((k_colfft<R, R, EF, NTS, true>), dim3((unsigned)nblocks), dim3(NTS), lds, st, jobs, blk0s,
-                           njobs);
-    else if (final)
-        hipLaunchKernelGGL((k_colfft<R, R, EF, NTF, true>), dim3((unsigned)nblocks), dim3(NTF), lds, st, jobs, blk0s,
-                           njobs);
+    const dim3 grid((unsigned)nblocks);
+    const int by_xcd = min_cols * (int)sizeof(typename cplx<R>::T) < 128 ? 1 : 0;
+    // the smallest final workgroup that holds every job's tile
+    if (!final)
+        hipLaunchKernelGGL((k_colfft<R, RY, EY, NTY, false>), grid, dim3(NTY), lds, st, jobs, blk0s, njobs,
+                           by_xcd);
+    else if (max_elems <= EF * NT0)
+        hipLaunchKernelGGL((k_colfft<R, R, EF, NT0, true>), grid, dim3(NT0), lds, st, jobs, blk0s, njobs,
+                           by_xcd);
+    else if (max_elems <= EF * NT1)
+        hipLaunchKernelGGL((k_colfft<R, R, EF, NT1, true>), grid, dim3(NT1), lds, st, jobs, blk0s, njobs,
+                           by_xcd);
     else
-        hipLaunchKernelGGL((k_colfft<R, RY, EY, NTY, false>), dim3((unsigned)nblocks), dim3(NTY), lds, st, jobs,
-                           blk0s, njobs);
+        hipLaunchKernelGGL((k_colfft<R, R, EF, NT2, true>), grid, dim3(NT2), lds, st, jobs, blk0s, njobs,
+                           by_xcd);
 }
 
 #define MPSQ_INST(R)                                                                                                  \
@@ -768,10 +793,10 @@ void launch_colfft_jobs(const ColJob<R> *jobs, const int *blk0s, int njobs, int 
     template void launch_gather<R>(int64_t, int, const int *, const cplx<R>::T *, cplx<R>::T *, int, hipStream_t);    \
     template void launch_binmax<R>(const PtRec<R> *, const int64_t *, const TransformInfo *, int, int, int *,         \
                                    hipStream_t);                                                                      \
-    template int colfft_tile_elems<R>(bool);                                                                          \
-    template int colfft_final_small_elems<R>();                                                                       \
+    template int colfft_max_len<R>();                                                                                 \
+    template int colfft_cols<R>(int64_t, int64_t, int64_t, bool);                                                     \
     template size_t colfft_lds<R>(const ColPass &, bool);                                                             \
-    template void launch_colfft_jobs<R>(const ColJob<R> *, const int *, int, int, bool, size_t, hipStream_t, int);
+    template void launch_colfft_jobs<R>(const ColJob<R> *, const int *, int, int, bool, size_t, hipStream_t, int, int);
 
 MPSQ_INST(float)
 MPSQ_INST(double)

@@ -1004,8 +1004,11 @@ __global__ __launch_bounds__(512, 4) void k_spread_wide(const SpreadJob<R> *__re
         const R beta = es_shape<R>(g.beta), ic = (R)g.ic;
         const C *tw = reinterpret_cast<const C *>(smem_raw + J.lds_tw);
         const float am = S.amax[pb];
+        // a pass that no point reaches (sparse inputs on fine grids) only
+        // writes zeros (FP32: unless the strengths are not finite)
+        const bool empty = total == 0 && !(F32 && !(am < 3.0e38f));
 
-        {
+        if (!empty) {
             uint4 *a4 = reinterpret_cast<uint4 *>(smem_raw);
             const int n16 = REAL ? pairs * RS : wplane;
             for (int i = threadIdx.x; i < n16; i += NT) a4[i] = make_uint4(0u, 0u, 0u, 0u);
@@ -1116,8 +1119,21 @@ __global__ __launch_bounds__(512, 4) void k_spread_wide(const SpreadJob<R> *__re
             cd.fetch(jobs[jn], S, pb ^ 1, vw + lane, tn, total_n, e);
         }
 
-        // ---- x FFT of the item's G rows
-        {
+        // grid row of pass row r
+        auto row_y = [&](int r, int &y, int &z) {
+            const int rz = P.bz > 1 ? (int)fdiv((uint32_t)r, J.dby) : 0;
+            y = P.y0 + r - rz * P.by;
+            z = P.z0 + rz;
+        };
+        if (empty) {
+            for (int r = wv; r < G; r += NT / 64) {
+                int y, z;
+                row_y(r, y, z);
+                C *gr = J.G1 + (((int64_t)t * g.n3 + z) * g.n2 + y) * J.g1_len;
+                for (int kk = lane; kk < J.g1_keep; kk += 64) gr[kk] = cmk<C>((R)0, (R)0);
+            }
+        } else {
+            // ---- x FFT of the item's G rows
             // cell a of a plane as a number (FP32: the low 48 bits of the
             // pattern sum); the ghost cells x = n1 + i fold onto i < w here
             auto cell = [&](int a, bool ghost) -> R {
@@ -1132,12 +1148,6 @@ __global__ __launch_bounds__(512, 4) void k_spread_wide(const SpreadJob<R> *__re
             };
             auto load_tile = [&](int row, int i) -> C { return tile[row * RSX + padx<true>(i)]; };
             auto store_tile = [&](int row, int i, C v) { tile[row * RSX + padx<true>(i)] = v; };
-            // grid row of pass row r
-            auto row_y = [&](int r, int &y, int &z) {
-                const int rz = P.bz > 1 ? (int)fdiv((uint32_t)r, J.dby) : 0;
-                y = P.y0 + r - rz * P.by;
-                z = P.z0 + rz;
-            };
             if constexpr (REAL) {
                 auto load_pair = [&](int pr, int i) -> C {
                     const int a = 2 * pr * RS + i;
