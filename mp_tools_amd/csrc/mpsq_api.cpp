@@ -1307,7 +1307,12 @@ template <typename R> struct Engine {
             return;
         }
         RadixPlan rp{};
-        const bool single = (p.n_frame == 1) && (T <= sqw_tile_elems<R>()) &&
+        // one window: direct DFT sums where they are fewer than the LDS FFT's
+        // fixed work (2.1 M columns, FP32: 16 frames to 8 frequencies 136 us
+        // against 348, 24 to 12 263 against 390, 32 to 16 388 against 407, 24
+        // to 24 426 against 420; FP64 alike), or none (S_tot alone)
+        const bool direct = p.n_f == 0 || T * p.n_f <= 400;
+        const bool single = (p.n_frame == 1) && !direct && (T <= sqw_tile_elems<R>()) &&
                             sqw_single_lds<R>(T, 1) <= SQW_MAX_LDS && radix_plan((int)T, rp);
         if (p.n_frame == 1) {
             if (win_n != (int)T || win_kind != r->win_kind) {
@@ -1337,7 +1342,7 @@ template <typename R> struct Engine {
             launch_sqw_single<R>(p, rpT, cols, amp, twT.as<Cx<R>>(), win_d.as<double>(), r->d_qfac, d_S, d_Stot, st);
             tm.end(ev, st);
         } else if (p.n_frame == 1) {
-            // one window, T without a radix plan: a DFT sum per frequency
+            // one window: a DFT sum per frequency
             dft_twiddles(p.n_int, st);
             const int ev = tm.begin(ST_REDUCE, st);
             launch_sqw_window1<R>(p, amp, r->d_qfac, win_d.as<double>(), twN.as<double2>(), d_S, d_Stot, st);

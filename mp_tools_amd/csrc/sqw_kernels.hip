@@ -12,8 +12,9 @@
 //                window is a sum of three exponentials) advanced by one frame
 //                per window; sum_s |X_s(m)|^2 accumulates in FP64
 //                (mp_sqom56.f90:1437-1478 computes the same sum per energy).
-// k_sqw_window1  one window over all frames when T has no 2,3,5 radix plan:
-//                DFT sums of a group of frequencies per wave.
+// k_sqw_window1  one window over all frames when T has no 2,3,5 radix plan or
+//                a short series needs few sums: DFT sums of a group of
+//                frequencies per wave.
 // k_iqt          I(Q,t) (mp_sqom56.f90:1467-1471, 1504-1510) by direct sums,
 //                a thread per Q and group of lags;
 // k_iqt_fft      the same for many lags by FFT correlation in LDS (FP64).
@@ -185,8 +186,8 @@ __device__ __forceinline__ void step_index(int &ix, int m, int n)
     if (ix >= n) ix -= n;
 }
 
-// One window over all T frames (n_frame == 1) when T has no 2,3,5 radix
-// plan: lane = Q, wave = group of MG frequencies,
+// One window over all T frames (n_frame == 1) by its definition (any T; the
+// host takes it where T has no 2,3,5 radix plan or the sums are few): lane = Q, wave = group of MG frequencies,
 //   X(m) = sum_i w_i C'(i) tw[(m i) mod n],  tw[k] = e^{-2 pi i k / n}.
 // The twiddles are the same for every Q, so they come from one table by
 // scalar loads and a frequency costs four FMAs per frame; a frame is read,
@@ -209,8 +210,8 @@ __global__ __launch_bounds__(256) void k_sqw_window1(SqwParams p, const typename
     amp += qs >= 0 ? qs : 0;  // lanes without a column read column 0 and write no value of it
     double mr = 0.0, mi = 0.0, ss = 0.0;
     if (p.subtract_mean || Stot) column_moments(amp, p.NQs, p.T, wv, nw, red, mr, mi, ss);
+    if (q < p.NQ && grp == 0 && Stot) Stot[q] = qs >= 0 ? ss * p.norm_tot : qnan();
     if (q >= p.NQ || grp * MG >= p.n_f) return;
-    if (grp == 0 && Stot) Stot[q] = qs >= 0 ? ss * p.norm_tot : qnan();
     if (!p.subtract_mean) mr = mi = 0.0;
     int m[MG], ix[MG];
     double dr[MG], di[MG];
@@ -319,11 +320,8 @@ __global__ __launch_bounds__(256, 4) void k_sqw_sliding(SqwParams p, const typen
     amp += qs >= 0 ? qs : 0;  // lanes without a column read column 0 and write no value of it
     double mr, mi, ss;
     column_moments(amp, p.NQs, p.T, wv, nw, red, mr, mi, ss);
-    if (q >= p.NQ || grp * MG >= p.n_f) {
-        if (q < p.NQ && grp == 0 && Stot) Stot[q] = qs >= 0 ? ss * p.norm_tot : qnan();
-        return;
-    }
-    if (grp == 0 && Stot) Stot[q] = qs >= 0 ? ss * p.norm_tot : qnan();
+    if (q < p.NQ && grp == 0 && Stot) Stot[q] = qs >= 0 ? ss * p.norm_tot : qnan();
+    if (q >= p.NQ || grp * MG >= p.n_f) return;
     if (!p.subtract_mean) mr = mi = 0.0;
     int m[MG], ix[MG];
     double Pr[MG], Pi[MG], Ur[MG], Ui[MG], Vr[MG], Vi[MG], acc[MG];
