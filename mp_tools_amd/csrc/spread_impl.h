@@ -178,10 +178,10 @@ template <typename R> size_t spread_tile_bytes(int by, int bz, int n1, int w, bo
     const size_t cb = sizeof(typename cplx<R>::T);
     if (real) {  // a wide pass of the real form: one 8-byte cell per row cell, FFT rows per pair
         const size_t pairs = (G + 1) / 2;
-        return (std::max(2 * pairs * RS * 8, pairs * RSX * cb) + 15) / 16 * 16;
+        return (std::max(2 * pairs * RS * 8 + (size_t)narrow_bias(w), pairs * RSX * cb) + 15) / 16 * 16;
     }
     const size_t narrowb = sizeof(R) == 4 ? rows * RSX * 8 + (size_t)narrow_bias(w) : 0;
-    const size_t wideb = std::max(2 * G * RS * 8, G * RSX * cb);
+    const size_t wideb = std::max(2 * G * RS * 8 + (size_t)narrow_bias(w), G * RSX * cb);
     return (std::max(narrowb, wideb) + 15) / 16 * 16;
 }
 template <typename R> size_t spread_lds_bytes(int by, int bz, int n1, int w, bool real)
@@ -954,8 +954,16 @@ __global__ __launch_bounds__(512, 4) void k_spread_wide(const SpreadJob<R> *__re
     const int vw = (NT / 64 - 1 - wv) * 64;
     const int xcd = blockIdx.x & 7;
     const int xbeg = fbl ? 0 : xr[xcd], xend = fbl ? wc[CTR_FB_COUNT] : xr[xcd + 1];
-    unsigned long long *acc64 = reinterpret_cast<unsigned long long *>(smem_raw);
-    double *accd = reinterpret_cast<double *>(smem_raw);
+    unsigned long long *acc64 = reinterpret_cast<unsigned long long *>(smem_raw + narrow_bias(W));
+    double *accd = reinterpret_cast<double *>(smem_raw + narrow_bias(W));
+    // lane order of a stencil's cells: rotated by lane group as in the narrow
+    // kernel (8-byte cells; a 10.5 M atom crystal to 512 x 512 x 64 in FP32
+    // 4.75 -> 3.36 ms a call, 320,000 atoms x 16 frames in FP64 4.30 -> 4.0)
+    constexpr int NG = (W >= 4) ? 4 : (W >= 2 ? 2 : 1), RSTEP = W / NG;
+    const int rg = lane & (NG - 1), rot = rg * RSTEP;
+    int rofs[NG];
+#pragma unroll
+    for (int s = 0; s < NG; ++s) rofs[s] = 8 * rot - ((rg >= NG - s) ? 8 * W : 0);
     C *tile = reinterpret_cast<C *>(smem_raw);
     // next item: its position k in [xbeg, xend) (k >= xend: none) -> tile id, pass
     auto take = [&]() -> int {
@@ -1009,7 +1017,7 @@ __global__ __launch_bounds__(512, 4) void k_spread_wide(const SpreadJob<R> *__re
         const bool empty = total == 0 && !(F32 && !(am < 3.0e38f));
 
         if (!empty) {
-            uint4 *a4 = reinterpret_cast<uint4 *>(smem_raw);
+            uint4 *a4 = reinterpret_cast<uint4 *>(acc64);
             const int n16 = REAL ? pairs * RS : wplane;
             for (int i = threadIdx.x; i < n16; i += NT) a4[i] = make_uint4(0u, 0u, 0u, 0u);
         }
@@ -1054,12 +1062,13 @@ __global__ __launch_bounds__(512, 4) void k_spread_wide(const SpreadJob<R> *__re
             if (g.dim >= 2) overlap(p.ly, P.y0, P.by, w, g.n2, fy, ny, my);
             if (g.dim >= 3) overlap(p.lz, P.z0, P.bz, w, g.n3, fz, nz, mz);
             if (ny <= 0 || nz <= 0) continue;
-            double kxd[W];
-            R kx[W];
+            // kx[m]: the kernel at the lane's m-th cell lx + (m + rot) mod W
+            double kx[W];
 #pragma unroll
             for (int m = 0; m < W; ++m) {
-                kx[m] = es_kernel(p.dx + (R)m, beta, ic);
-                kxd[m] = (double)kx[m] * fscale;
+                const int mm = (m + rot < W) ? m + rot : m + rot - W;
+                kx[m] = (double)es_kernel(p.dx + (R)mm, beta, ic);
+                if (F32) kx[m] *= fscale;
             }
             R ky[W];
 #pragma unroll
@@ -1075,30 +1084,42 @@ __global__ __launch_bounds__(512, 4) void k_spread_wide(const SpreadJob<R> *__re
                 for (int iy = 0; iy < W; ++iy) {
                     if (iy < nyb && iy < ny) {
                         const R wyz = ky[iy] * wz;
-                        const int c0 = __mul24(rr0 + iy, RS) + p.lx;
-                        if (F32) {
+                        unsigned char *ab = reinterpret_cast<unsigned char *>(acc64 + (__mul24(rr0 + iy, RS) + p.lx));
+                        unsigned char *base[NG];
+#pragma unroll
+                        for (int s = 0; s < NG; ++s) base[s] = ab + rofs[s];
+                        // the lane's m-th cell; groups g >= NG - seg have wrapped
+                        auto cell = [&](int m) -> unsigned char * {
+                            int seg = 0;
+#pragma unroll
+                            for (int q = 1; q < NG; ++q) seg += (m >= W - q * RSTEP) ? 1 : 0;
+                            return base[seg] + 8 * m;
+                        };
+                        auto add64 = [&](unsigned char *a, unsigned long long x) {
+                            __hip_atomic_fetch_add(reinterpret_cast<unsigned long long *>(a), x, __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+                        };
+                        auto addd = [&](unsigned char *a, double x) {
+                            __hip_atomic_fetch_add(reinterpret_cast<double *>(a), x, __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+                        };
+                        const int wplane_b = wplane * 8;
+                        if constexpr (F32) {
                             const double vr = (double)(cc.x * wyz), vi = (double)(cc.y * wyz);
-                            unsigned long long *ar = acc64 + c0, *ai = acc64 + wplane + c0;
 #pragma unroll
                             for (int m = 0; m < W; ++m) {
-                                const double dr = __builtin_fma(vr, kxd[m], FIX_MAGIC);
-                                __hip_atomic_fetch_add(ar + m, (unsigned long long)__double_as_longlong(dr),
-                                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                                if constexpr (REAL) continue;
-                                const double di = __builtin_fma(vi, kxd[m], FIX_MAGIC);
-                                __hip_atomic_fetch_add(ai + m, (unsigned long long)__double_as_longlong(di),
-                                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                                add64(cell(m), (unsigned long long)__double_as_longlong(
+                                                   __builtin_fma(vr, kx[m], FIX_MAGIC)));
+                                if constexpr (!REAL)
+                                    add64(cell(m) + wplane_b, (unsigned long long)__double_as_longlong(
+                                                                  __builtin_fma(vi, kx[m], FIX_MAGIC)));
                             }
                         } else {
-                            const R vr = cc.x * wyz, vi = cc.y * wyz;
-                            double *ar = accd + c0, *ai = accd + wplane + c0;
+                            const double vr = cc.x * wyz, vi = cc.y * wyz;
 #pragma unroll
                             for (int m = 0; m < W; ++m) {
-                                __hip_atomic_fetch_add(ar + m, (double)(vr * kx[m]), __ATOMIC_RELAXED,
-                                                       __HIP_MEMORY_SCOPE_WORKGROUP);
-                                if constexpr (REAL) continue;
-                                __hip_atomic_fetch_add(ai + m, (double)(vi * kx[m]), __ATOMIC_RELAXED,
-                                                       __HIP_MEMORY_SCOPE_WORKGROUP);
+                                addd(cell(m), vr * kx[m]);
+                                if constexpr (!REAL) addd(cell(m) + wplane_b, vi * kx[m]);
                             }
                         }
                     }
