@@ -302,11 +302,22 @@ struct Arena {
     DevBuf d;
     hipEvent_t ev = nullptr;
     bool pending = false;
+    // what the device has: the first `sent` bytes, uploaded on sent_st; tables
+    // equal to it (a plan's next points, an engine's next batch of frames) are
+    // not uploaded again
+    size_t sent = 0;
+    hipStream_t sent_st = nullptr;
+    bool dirty = true;
     void begin()
+    {
+        used = 0;
+        dirty = sent == 0;
+    }
+    void touch()
     {
         if (pending) HIPCHK(hipEventSynchronize(ev));
         pending = false;
-        used = 0;
+        dirty = true;
     }
     size_t put_raw(const void *src, size_t bytes)
     {
@@ -314,6 +325,7 @@ struct Arena {
         if (off + bytes > cap) {
             size_t nc = std::max<size_t>(cap * 2, 1 << 16);
             while (nc < off + bytes) nc *= 2;
+            touch();
             unsigned char *nh = nullptr;
             HIPCHK(hipHostMalloc(reinterpret_cast<void **>(&nh), nc, hipHostMallocDefault));
             if (h) {
@@ -323,19 +335,25 @@ struct Arena {
             h = nh;
             cap = nc;
         }
-        if (bytes) std::memcpy(h + off, src, bytes);
+        if (bytes && (dirty || off + bytes > sent || std::memcmp(h + off, src, bytes) != 0)) {
+            if (!dirty || pending) touch();
+            std::memcpy(h + off, src, bytes);
+        }
         used = off + bytes;
         return off;
     }
     template <typename T> size_t put(const std::vector<T> &v) { return put_raw(v.data(), sizeof(T) * v.size()); }
     void upload(hipStream_t st)
     {
-        if (used == 0) return;
+        if (used == 0 || (!dirty && used <= sent && st == sent_st)) return;
+        sent = 0;
         d.ensure(used);
         if (!ev) HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
         HIPCHK(hipMemcpyAsync(d.p, h, used, hipMemcpyHostToDevice, st));
         HIPCHK(hipEventRecord(ev, st));
         pending = true;
+        sent = used;
+        sent_st = st;
     }
     template <typename T> const T *dev(size_t off) const
     {
@@ -421,7 +439,8 @@ template <typename R> struct Core {
     bool real = false;
     int rows_max = 1;
 
-    void setup(int dim_, const int64_t *nm, int iflag_, double eps_, const mpsq_opts *o, bool real_ = false)
+    // ntr: transforms of a run, where they are known (0: not)
+    void setup(int dim_, const int64_t *nm, int iflag_, double eps_, const mpsq_opts *o, bool real_ = false, int ntr = 0)
     {
         if (dim_ < 1 || dim_ > 3 || !nm) throw Err{MPSQ_ERR_BAD_ARG};
         dim = dim_;
@@ -483,6 +502,11 @@ template <typename R> struct Core {
         int rows_def = rows_max;
         while (real && sizeof(R) == 8 && rows_def > 2 && spread_lds<R>(rows_def, 1, (int)n[0], w, true) > 80 * 1024)
             rows_def /= 2;
+        // grids of few rows: tiles of fewer rows, so that every workgroup the
+        // chip holds at once (two per CU) has one (48 x 40 x 24 cells, 2,000
+        // points: 15 tiles of 64 rows 53 us, 480 of 2 rows 17 us; 320 x 320,
+        // 32,768 points: 40 of 8 rows 38 us, 320 of one row 23 us)
+        while (sizeof(R) == 8 && ntr > 0 && rows_def > 1 && n[1] * n[2] / rows_def * ntr < 256) rows_def /= 2;
         const int bmax = spread_max_tile_b();
         int by = 1, bz = 1;
         if (dim == 2) {
@@ -713,10 +737,16 @@ template <typename R> struct Plan {
     Core<R> core;
     int ntrans = 1;
     int64_t M = -1;
-    DevBuf xyz[3], rec, key, srec, perm, H, Hs, bsum, binstart, binmax, bad, wc, fbl;
+    DevBuf xyz[3], rec, key, srec, perm, H, Hs, bsum, binstart, binmax, wc, fbl;
     DevBuf cin, cs, G1, G2, fout, amax;
     Arena sort_tab, run_tab;
+    int *bad_h = nullptr;  // non-finite point seen by the last setpts: host memory the fold writes
     int nch = 0;
+    ~Plan()
+    {
+        if (core.st) (void)hipStreamSynchronize(core.st);
+        if (bad_h) (void)hipHostFree(bad_h);
+    }
     size_t off_chunks = 0, off_tinfo = 0;
 
     void setpts(int64_t M_, const R *x, const R *y, const R *z, bool on_device)
@@ -743,10 +773,6 @@ template <typename R> struct Plan {
         srec.ensure(sizeof(PtRec<R>) * Mb);
         key.ensure(sizeof(int) * Mb);
         perm.ensure(sizeof(int) * Mb);
-        bad.ensure(sizeof(int));
-        HIPCHK(hipMemsetAsync(bad.p, 0, sizeof(int), c.st));
-        launch_fold<R>(c.g, M_, dptr[0], dptr[1], dptr[2], sizeof(R) == 4, rec.as<PtRec<R>>(), key.as<int>(),
-                       bad.as<int>(), c.st);
         const int64_t CH = c.sort_chunk;
         nch = (int)((M_ + CH - 1) / CH);
         std::vector<SortChunk> chunks((size_t)std::max(nch, 1));
@@ -778,23 +804,29 @@ template <typename R> struct Plan {
         Hs.ensure(sizeof(int64_t) * (size_t)std::max<int64_t>(Htot, 1));
         bsum.ensure(sizeof(int64_t) * (size_t)scan_bsum_size(Htot));
         binstart.ensure(sizeof(int64_t) * (size_t)(c.g.nbins + 1));
+        if (sizeof(R) == 4) binmax.ensure(sizeof(int) * (size_t)(c.g.nbins + 1));
         const SortChunk *chd = sort_tab.dev<SortChunk>(off_chunks);
+        if (!bad_h) HIPCHK(hipHostMalloc(reinterpret_cast<void **>(&bad_h), sizeof(int), hipHostMallocDefault));
+        *bad_h = 0;  // (nothing below throws before this call has waited for its kernels)
+        launch_fold<R>(c.g, M_, dptr[0], dptr[1], dptr[2], sizeof(R) == 4, rec.as<PtRec<R>>(), key.as<int>(), bad_h,
+                       c.st);
         launch_sort_count(key.as<int>(), chd, nch, c.g.nbins, H.as<int>(), c.st);
-        launch_scan(H.as<int>(), Htot, bsum.as<int64_t>(), Hs.as<int64_t>(), c.st);
+        const bool small = launch_scan_small(H.as<int>(), c.g.nbins, nch, M_, Hs.as<int64_t>(), binstart.as<int64_t>(),
+                                             c.st);
+        if (!small) launch_scan(H.as<int>(), Htot, bsum.as<int64_t>(), Hs.as<int64_t>(), c.st);
         launch_sort_scatter<R>(key.as<int>(), chd, nch, c.g.nbins, Hs.as<int64_t>(), rec.as<PtRec<R>>(), nullptr,
                                srec.as<PtRec<R>>(), nullptr, perm.as<int>(), c.st);
-        launch_binstart(Hs.as<int64_t>(), sort_tab.dev<TransformInfo>(off_tinfo), 1, c.g.nbins,
+        if (!small)
+            launch_binstart(Hs.as<int64_t>(), sort_tab.dev<TransformInfo>(off_tinfo), 1, c.g.nbins,
                         binstart.as<int64_t>(), c.st);
         if (sizeof(R) == 4) {
-            binmax.ensure(sizeof(int) * (size_t)(c.g.nbins + 1));
             launch_binmax<R>(srec.as<PtRec<R>>(), binstart.as<int64_t>(), sort_tab.dev<TransformInfo>(off_tinfo), 1,
                              c.g.nbins, binmax.as<int>(), c.st);
         }
-        HIPCHK(hipGetLastError());
-        int hbad = 0;
-        HIPCHK(hipMemcpyAsync(&hbad, bad.p, sizeof(int), hipMemcpyDeviceToHost, c.st));
+        const hipError_t le = hipGetLastError();
         HIPCHK(hipStreamSynchronize(c.st));
-        throw_bad(hbad);
+        HIPCHK(le);
+        throw_bad(*bad_h);
         M = M_;
     }
 
@@ -835,9 +867,11 @@ template <typename R> struct Plan {
             launch_absmax(M, ntrans, reinterpret_cast<const float2 *>(cs.p), amax.as<float>(), c.st);
             am = amax.as<float>();
         }
-        // one-entry job tables: spread, then the column passes
-        launch_zero_i32(bad.as<int>(), 1, c.st);
-        std::vector<SpreadJob<R>> sj(1, c.spreadjob(ntrans, srec.as<PtRec<R>>(), M, bad.as<int>(), cs.as<Cx<R>>(), M,
+        // one-entry job tables: spread, then the column passes (the error
+        // flag is a spare counter, which the spread's launch clears with the rest)
+        wc.ensure(sizeof(int) * XCD_CTR_INTS);
+        int *err = wc.as<int>() + XCD_CTR_INTS - 1;
+        std::vector<SpreadJob<R>> sj(1, c.spreadjob(ntrans, srec.as<PtRec<R>>(), M, err, cs.as<Cx<R>>(), M,
                                                      binstart.as<int64_t>(),
                                                      sizeof(R) == 4 ? binmax.as<int>() : nullptr, 0, g1, am,
                                                      (c.dim == 1 && c.iflag > 0) ? 1 : 0));
@@ -855,7 +889,6 @@ template <typename R> struct Plan {
         const size_t o_sj = run_tab.put(sj), o_z = run_tab.put(zero1), o_xr = run_tab.put(xr);
         const size_t o_cy = run_tab.put(cy), o_cz = run_tab.put(cz);
         run_tab.upload(c.st);
-        wc.ensure(sizeof(int) * XCD_CTR_INTS);
         fbl.ensure(sizeof(int) * (size_t)spread_max_wide_passes() * (size_t)ntile);
         launch_spread_jobs<R>(run_tab.dev<SpreadJob<R>>(o_sj), run_tab.dev<int>(o_z), 1, c.g.w,
                               run_tab.dev<int>(o_xr), wc.as<int>(), fbl.as<int>(), c.spread_lds_size(), c.st);
@@ -870,7 +903,7 @@ template <typename R> struct Plan {
         HIPCHK(hipGetLastError());
         if (!on_device) {
             int hbad = 0;
-            HIPCHK(hipMemcpyAsync(&hbad, bad.p, sizeof(int), hipMemcpyDeviceToHost, c.st));
+            HIPCHK(hipMemcpyAsync(&hbad, err, sizeof(int), hipMemcpyDeviceToHost, c.st));
             HIPCHK(hipMemcpyAsync(f_out, fd, sizeof(Cx<R>) * (size_t)NQ * ntrans, hipMemcpyDeviceToHost, c.st));
             HIPCHK(hipStreamSynchronize(c.st));
             throw_bad(hbad);
@@ -901,7 +934,7 @@ template <typename R> static int makeplan_impl(int type, int dim, const int64_t 
     if (!p) return MPSQ_ERR_DEVICE;
     try {
         p->ntrans = ntrans;
-        p->core.setup(dim, nm, iflag, eps, o);
+        p->core.setup(dim, nm, iflag, eps, o, false, ntrans);
     } catch (const Err &e) {
         delete p;
         return e.code;
@@ -1800,7 +1833,7 @@ template <typename R> struct Batch {
         if (use_graph && key == gkey && !gexec) {
             // capture: everything is allocated and the tables are current
             HIPCHK(hipStreamSynchronize(st));
-            for (Arena *a : arenas) a->begin();  // nothing pending may be waited on inside the capture
+            for (Arena *a : arenas) a->touch();  // nothing pending may be waited on inside the capture
             HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
             enqueue(d_pos, T, d_amp, r, d_S, d_Stot, nullptr);
             hipGraph_t g = nullptr;

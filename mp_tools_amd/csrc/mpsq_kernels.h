@@ -185,6 +185,9 @@ void launch_stage_jobs(const StageJob *jobs, const int *blk0s, int njobs, int nb
                        typename cplx<R>::T *cstr, int *bad, hipStream_t st);
 void launch_sort_count(const int *key, const SortChunk *chunks, int nchunks, int max_nbins, int *H, hipStream_t st);
 void launch_scan(const int *H, int64_t n, int64_t *bsum, int64_t *Hs, hipStream_t st);
+// one transform's scan and bin starts in one launch; false (nothing done) if
+// its count matrix is too large for that
+bool launch_scan_small(const int *H, int nbins, int nch, int64_t M, int64_t *Hs, int64_t *binstart, hipStream_t st);
 int64_t scan_bsum_size(int64_t n);
 template <typename R>
 void launch_sort_scatter(const int *key, const SortChunk *chunks, int nchunks, int max_nbins, const int64_t *Hs,
