@@ -38,6 +38,13 @@ __device__ __forceinline__ void fold1(double xv, double s, double hw, int n, int
     const double t = u - hw;
     const double lf = ceil(t);
     d = lf - u;
+    // within a period of the grid (every folded coordinate): no 64-bit modulo
+    // (staging 41 M points of 128 frames: 620 us with it alone, 469 so)
+    if (fabs(lf) < (double)n) {
+        const int li = (int)lf;
+        l = li < 0 ? li + n : li;
+        return;
+    }
     long long lw = 0;
     if (isfinite(lf) && fabs(lf) < 9.0e18) lw = (long long)lf;
     else bad = 1;
