@@ -2256,7 +2256,8 @@ static void dos_run(const float *d_vel, int64_t T, int64_t n_tot, const int32_t 
     p.norm_s = 1.0 / (double)T;
     p.norm_tot = 0.0;
     RadixPlan rp{};
-    const bool single = (T <= sqw_tile_elems<R>()) && dos_fused_lds<R>(T, 1) <= SQW_MAX_LDS && radix_plan((int)T, rp);
+    const bool single = (T <= sqw_tile_elems<R>()) && dos_fused_lds<R>(T, 1) <= SQW_MAX_LDS && dos_fused_ok<R>(n_freq) &&
+                        radix_plan((int)T, rp);
     DevBuf tw, win, S, buf;
     int cols = 1;
     std::vector<double> wh((size_t)T);
@@ -2274,28 +2275,22 @@ static void dos_run(const float *d_vel, int64_t T, int64_t n_tot, const int32_t 
     }
     launch_zero_i32(reinterpret_cast<int *>(d_dos), (int)(2 * n_freq * nsp), st);
     if (single) {
-        // one pass: FFT, |X|^2 and per-block species sums (no |FFT|^2 rows
-        // in HBM); blocks per launch keep their sums within 256 MB
+        // one pass: FFT, |X|^2 and per-block species sums (no |FFT|^2 rows in HBM)
         const int64_t nout = (int64_t)nsp * n_freq;
-        const int64_t nblk = (ncs + cols - 1) / cols;
-        const int64_t bpl = std::max<int64_t>(1, std::min<int64_t>(nblk, ((int64_t)256 << 20) / (8 * nout)));
+        const int64_t rows = dos_fused_rows<R>((ncs + cols - 1) / cols, n_freq);
         DevBuf part;
-        part.ensure(sizeof(double) * (size_t)((bpl + dos_reduce_groups()) * nout));
+        part.ensure(sizeof(double) * (size_t)((rows + dos_reduce_groups()) * nout));
         DosParams dp{};
         dp.T = T;
         dp.ncs = ncs;
+        dp.c0 = 0;
+        dp.nc = ncs;
         dp.n_freq = n_freq;
         dp.nsp = nsp;
         dp.norm = 1.0 / (double)T;
-        for (int64_t b0 = 0; b0 < nblk; b0 += bpl) {
-            const int64_t nb = std::min(bpl, nblk - b0);
-            dp.c0 = b0 * cols;
-            dp.nc = std::min(nb * cols, ncs - dp.c0);
-            launch_dos_fused<R>(dp, rp, cols, d_vel, d_at_ind, tw.as<Cx<R>>(), win.as<double>(), part.as<double>(),
-                                st);
-            dos_reduce_parts(part.as<double>(), nb, nsp, (int)n_freq, part.as<double>() + bpl * nout, d_dos, st);
-            HIPCHK(hipGetLastError());
-        }
+        launch_dos_fused<R>(dp, rp, cols, d_vel, d_at_ind, tw.as<Cx<R>>(), win.as<double>(), part.as<double>(), st);
+        dos_reduce_parts(part.as<double>(), rows, nsp, (int)n_freq, part.as<double>() + rows * nout, d_dos, st);
+        HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(st));
         return;
     }

@@ -225,12 +225,12 @@ __host__ __device__ inline int padded_len(int n) { return n + (n >> 4) + 1; }
 // take consecutive butterflies of one transform (es == 1, rows may be padded).
 template <typename C, int E, int R, bool PAD>
 __device__ __forceinline__ void stockham_stage(C *buf, int n, int cnt, FDiv dcnt, FDiv dnb, FDiv dns, int es, int ts,
-                                               int Ns, const C *__restrict__ tw, bool col_major)
+                                               int Ns, const C *__restrict__ tw, bool col_major, int tid)
 {
     constexpr int TPT = (E + R - 1) / R;
     const int nb = n / R;
     const int total = nb * cnt;
-    const int tid = threadIdx.x, NT = blockDim.x;
+    const int NT = blockDim.x;
     const int tstride = n / (Ns * R);
     C v[TPT * R];
     int tt[TPT], jj[TPT];
@@ -276,26 +276,64 @@ __device__ __forceinline__ void stockham_stage(C *buf, int n, int cnt, FDiv dcnt
     __syncthreads();
 }
 
+// Time columns held in registers, frames seg + k * nseg (k < E) of column c in
+// v[k], to the [T][cols] tile.  Where the tile is full (T = E * nseg) and the
+// first radix is 8, a thread's elements are E / 8 whole butterflies of the
+// first stage (inputs T / 8 = (E / 8) nseg frames apart): the stage runs here,
+// without the tile's write and read before it.  Returns the stages done.
+template <typename C, int E>
+__device__ __forceinline__ int stage_from_registers(C (&v)[E], C *tile, const RadixPlan &rp, int T, int cols, int c,
+                                                    int seg, int nseg)
+{
+    if (T == E * nseg && rp.r[0] == 8) {
+        constexpr int M = E / 8;
+#pragma unroll
+        for (int j = 0; j < M; ++j) {
+            C a[8];
+#pragma unroll
+            for (int r = 0; r < 8; ++r) a[r] = v[j + r * M];
+            Bfly<8, C>::run(a);
+            const int b = (seg + j * nseg) * 8;
+#pragma unroll
+            for (int r = 0; r < 8; ++r) tile[(b + r) * cols + c] = a[r];
+        }
+        return 1;
+    }
+#pragma unroll
+    for (int k = 0; k < E; ++k)
+        if (seg + k * nseg < T) tile[(seg + k * nseg) * cols + c] = v[k];
+    return 0;
+}
+
 // Full forward FFT of the tile (natural order in, natural order out).
-// dcnt = make_fdiv(cnt) (used in col_major mode).
+// dcnt = make_fdiv(cnt) (used in col_major mode).  tid: threadIdx.x, or a copy
+// the compiler cannot see through, for a caller that loops over tiles (else
+// it keeps every stage's index arithmetic in registers across the loop).
+// s0: stages already done (stage_from_registers).
 template <typename C, int E, bool PAD = false>
 __device__ __forceinline__ void lds_fft(C *buf, const RadixPlan &rp, int cnt, FDiv dcnt, int es, int ts, const C *__restrict__ tw,
-                        bool col_major)
+                        bool col_major, int tid, int s0 = 0)
 {
-    int Ns = 1;
-    for (int s = 0; s < rp.nst; ++s) {
+    int Ns = s0 > 0 ? rp.r[0] : 1;
+    for (int s = s0; s < rp.nst; ++s) {
         const int R = rp.r[s];
         const FDiv dnb = rp.dnb[s], dns = rp.dns[s];
         switch (R) {
-        case 8: stockham_stage<C, E, 8, PAD>(buf, rp.n, cnt, dcnt, dnb, dns, es, ts, Ns, tw, col_major); break;
-        case 4: stockham_stage<C, E, 4, PAD>(buf, rp.n, cnt, dcnt, dnb, dns, es, ts, Ns, tw, col_major); break;
-        case 2: stockham_stage<C, E, 2, PAD>(buf, rp.n, cnt, dcnt, dnb, dns, es, ts, Ns, tw, col_major); break;
-        case 3: stockham_stage<C, E, 3, PAD>(buf, rp.n, cnt, dcnt, dnb, dns, es, ts, Ns, tw, col_major); break;
-        case 5: stockham_stage<C, E, 5, PAD>(buf, rp.n, cnt, dcnt, dnb, dns, es, ts, Ns, tw, col_major); break;
+        case 8: stockham_stage<C, E, 8, PAD>(buf, rp.n, cnt, dcnt, dnb, dns, es, ts, Ns, tw, col_major, tid); break;
+        case 4: stockham_stage<C, E, 4, PAD>(buf, rp.n, cnt, dcnt, dnb, dns, es, ts, Ns, tw, col_major, tid); break;
+        case 2: stockham_stage<C, E, 2, PAD>(buf, rp.n, cnt, dcnt, dnb, dns, es, ts, Ns, tw, col_major, tid); break;
+        case 3: stockham_stage<C, E, 3, PAD>(buf, rp.n, cnt, dcnt, dnb, dns, es, ts, Ns, tw, col_major, tid); break;
+        case 5: stockham_stage<C, E, 5, PAD>(buf, rp.n, cnt, dcnt, dnb, dns, es, ts, Ns, tw, col_major, tid); break;
         default: break;
         }
         Ns *= R;
     }
+}
+template <typename C, int E, bool PAD = false>
+__device__ __forceinline__ void lds_fft(C *buf, const RadixPlan &rp, int cnt, FDiv dcnt, int es, int ts, const C *__restrict__ tw,
+                        bool col_major)
+{
+    lds_fft<C, E, PAD>(buf, rp, cnt, dcnt, es, ts, tw, col_major, (int)threadIdx.x);
 }
 
 }  // namespace mpsq

@@ -735,18 +735,33 @@ void launch_dos_species(const double *S, int64_t ncols, int64_t c0, int64_t n_fr
                        reinterpret_cast<const int4 *>(at_ind), nsp, dos);
 }
 
-// The same spectra without the |FFT|^2 rows in HBM: a block loads `cols`
-// packed velocity columns (first column c0 + block * cols), applies the
-// window, runs the time FFT in LDS like k_sqw_single, and for every atom type
-// s and frequency f writes
-//   part[block][s][f] = sum over its columns of type s, in column order, of
-//                       (|X(f)|^2 + |X(-f)|^2) / 2 * norm
-// (FP64); dos_reduce_parts adds the blocks' rows in a fixed order.
-template <typename R, int E, int NT>
-__global__ __launch_bounds__(NT) void k_dos_fused(DosParams p, RadixPlan rp, int cols, FDiv dcols,
-                                                  const float2 *__restrict__ vel, const int4 *__restrict__ at_ind,
-                                                  const typename cplx<R>::T *__restrict__ tw,
-                                                  const double *__restrict__ win, double *__restrict__ part)
+// v as the registers hold it now: orders the steps on either side, so that
+// the FP64 copies of a thread's elements are not all alive at once
+template <typename C> __device__ __forceinline__ void pin(C &v) { asm volatile("" : "+v"(v.x), "+v"(v.y)); }
+
+// The same spectra without the |FFT|^2 rows in HBM: a block walks groups of
+// `cols` packed velocity columns (first column c0 + group * cols; groups
+// block, block + grid, ...), applies the window, runs the time FFT in LDS like
+// k_sqw_single, and adds for every frequency f, over the group's columns,
+//   (|X(f)|^2 + |X(-f)|^2) / 2 * norm
+// in FP64 registers: thread (f, h) the columns h, h + nh, ..., from one that
+// depends on f so that lanes read different LDS banks (nh = NT / n_freq
+// shares of the columns; beyond NT frequencies a thread holds several).  The
+// sums belong to the atom type the columns are of; when it changes (groups of
+// several types: for each in turn) they go to the row of share h,
+// part[block * nh + h][type][f], and start again.  dos_reduce_parts adds the
+// rows in a fixed order.  At most 128 registers: two workgroups per CU.
+// (640,000 columns of 512 frames, 5 types x 256 frequencies, with a row per
+// group and a test of every column per type and frequency: 2 x 841 us and 2 x
+// 131 us for its 410 MB of rows; now 1584 us in one launch.)
+// KO: frequencies per thread (1 while n_freq <= NT)
+constexpr int DOS_ACC = 9;
+template <typename R, int E, int NT, int KO>
+__global__ __launch_bounds__(NT, 4) void k_dos_fused(DosParams p, RadixPlan rp, int cols, FDiv dcols, FDiv dnf, int nh,
+                                                     int ngroups, const float2 *__restrict__ vel,
+                                                     const int4 *__restrict__ at_ind,
+                                                     const typename cplx<R>::T *__restrict__ tw,
+                                                     const double *__restrict__ win, double *__restrict__ part)
 {
     using C = typename cplx<R>::T;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -755,44 +770,107 @@ __global__ __launch_bounds__(NT) void k_dos_fused(DosParams p, RadixPlan rp, int
     C *tw_l = tile + T * cols;
     __shared__ int spc[SQW_MAX_COLS];
     for (int i = threadIdx.x; i < T; i += NT) tw_l[i] = tw[i];
-    const int64_t q0 = p.c0 + (int64_t)blockIdx.x * cols;
-    const int ncol = (int)min((int64_t)cols, p.c0 + p.nc - q0);
-    if ((int)threadIdx.x < cols) spc[threadIdx.x] = (int)threadIdx.x < ncol ? at_ind[(q0 + threadIdx.x) >> 1].w - 1 : -1;
-    {
-        C v[E];
-#pragma unroll
-        for (int k = 0; k < E; ++k) {
-            const int i = threadIdx.x + k * NT;
-            const int t = (int)fdiv((uint32_t)i, dcols), c = i - t * cols;
-            v[k] = cmk<C>((R)0, (R)0);
-            if (i < T * cols && c < ncol) {
-                const float2 a = vel[(int64_t)t * p.ncs + q0 + c];
-                const double w = win[t];
-                v[k] = cmk<C>((R)((double)a.x * w), (R)((double)a.y * w));
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < E; ++k) {
-            const int i = threadIdx.x + k * NT;
-            if (i < T * cols) tile[i] = v[k];
-        }
-    }
-    __syncthreads();
-    lds_fft<C, E>(tile, rp, cols, dcols, cols, 1, tw_l, true);
     const int nf = (int)p.n_freq, nout = p.nsp * nf;
-    double *dst = part + (int64_t)blockIdx.x * nout;
-    for (int i = threadIdx.x; i < nout; i += NT) {
-        const int s = i / nf, f = i - s * nf;
-        const int fm = f == 0 ? 0 : T - f;
-        double acc = 0.0;
-        for (int c = 0; c < ncol; ++c)
-            if (spc[c] == s) {
-                const C a = tile[f * cols + c], b = tile[fm * cols + c];
-                acc += 0.5 * (((double)a.x * (double)a.x + (double)a.y * (double)a.y) * p.norm +
-                              ((double)b.x * (double)b.x + (double)b.y * (double)b.y) * p.norm);
+    const int h = nh > 1 ? (int)fdiv((uint32_t)threadIdx.x, dnf) : 0;
+    const int f0 = (int)threadIdx.x - h * nf;  // first frequency (nh == 1: then every NT-th)
+    const bool own = h < nh && f0 < nf;
+    const int ns = own ? (cols - h + nh - 1) / nh : 0;  // columns of the share in a whole group
+    const int rot = ns > 0 ? f0 % ns : 0;
+    double *row = part + (int64_t)(blockIdx.x * nh + h) * nout;
+    double acc[KO];
+#pragma unroll
+    for (int k = 0; k < KO; ++k) acc[k] = 0.0;
+    if (own)
+        for (int f = f0; f < nf; f += NT)
+            for (int s = 0; s < p.nsp; ++s) row[s * nf + f] = 0.0;
+    int cur = -1;  // type the sums are of
+    auto flush = [&]() {
+#pragma unroll
+        for (int k = 0; k < KO; ++k) {
+            const int f = f0 + k * NT;
+            if (own && f < nf && cur >= 0) row[cur * nf + f] += acc[k] * (0.5 * p.norm);
+            acc[k] = 0.0;
+        }
+    };
+    for (int g = blockIdx.x; g < ngroups; g += gridDim.x) {
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));  // (see lds_fft)
+        const int64_t q0 = p.c0 + (int64_t)g * cols;
+        const int ncol = (int)min((int64_t)cols, p.c0 + p.nc - q0);
+        // NT is a multiple of cols: a thread's elements are column c0, frames
+        // seg, seg + nseg, ...
+        const int seg = (int)fdiv((uint32_t)tid, dcols), c0 = tid - seg * cols, nseg = NT / cols;
+        if (tid < cols) {
+            // types outside [0, nsp) count for nothing
+            const int s = tid < ncol ? at_ind[(q0 + tid) >> 1].w - 1 : -1;
+            spc[tid] = s >= 0 && s < p.nsp ? s : -1;
+        }
+        int done;
+        {
+            // all loads of a thread in flight before any use
+            float2 a[E];
+            const float2 *src = vel + q0 + c0;
+#pragma unroll
+            for (int k = 0; k < E; ++k) {
+                const int t = seg + k * nseg;
+                a[k] = make_float2(0.0f, 0.0f);
+                if (t < T && c0 < ncol) a[k] = src[(int64_t)t * p.ncs];
             }
-        dst[i] = acc;
+            C v[E];
+#pragma unroll
+            for (int k = 0; k < E; ++k) {
+                const double w = seg + k * nseg < T ? win[seg + k * nseg] : 0.0;
+                v[k] = cmk<C>((R)((double)a[k].x * w), (R)((double)a[k].y * w));
+                pin(v[k]);
+            }
+            done = stage_from_registers<C, E>(v, tile, rp, T, cols, c0, seg, nseg);
+        }
+        __syncthreads();
+        lds_fft<C, E>(tile, rp, cols, dcols, cols, 1, tw_l, true, tid, done);
+        // the group's types, each after the one before it in column order
+        for (int cs = 0; cs < ncol;) {
+            const int s = __builtin_amdgcn_readfirstlane(spc[cs]);
+            int ce = cs + 1;  // columns [cs, ce) are of type s
+            while (ce < ncol && __builtin_amdgcn_readfirstlane(spc[ce]) == s) ++ce;
+            if (s >= 0) {
+                if (s != cur) {
+                    flush();
+                    cur = s;
+                }
+                if (own) {
+#pragma unroll
+                    for (int k = 0; k < KO; ++k) {
+                        const int f = f0 + k * NT;
+                        if (k * NT >= nf) break;  // uniform
+                        if (f >= nf) continue;
+                        const C *ta = tile + f * cols, *tb = tile + (f == 0 ? 0 : T - f) * cols;
+                        double x = acc[k];
+                        auto add = [&](int c) {
+                            const C a = ta[c], b = tb[c];
+                            x += ((double)a.x * (double)a.x + (double)a.y * (double)a.y) +
+                                 ((double)b.x * (double)b.x + (double)b.y * (double)b.y);
+                        };
+                        if (ce - cs == cols) {
+                            // a whole group: lane f starts at column f mod ns of
+                            // its share (rows are a multiple of the banks apart)
+                            int i = rot;
+#pragma unroll 4
+                            for (int n = 0; n < ns; ++n) {
+                                add(h + i * nh);
+                                if (++i == ns) i = 0;
+                            }
+                        } else {
+                            for (int c = cs + h; c < ce; c += nh) add(c);
+                        }
+                        acc[k] = x;
+                    }
+                }
+            }
+            cs = ce;
+        }
+        __syncthreads();
     }
+    flush();
 }
 
 template <typename R> size_t dos_fused_lds(int64_t T, int cols)
@@ -800,22 +878,50 @@ template <typename R> size_t dos_fused_lds(int64_t T, int cols)
     return (size_t)T * (size_t)(cols + 1) * sizeof(typename cplx<R>::T);
 }
 
+// shares of the columns: threads per frequency
+template <typename R> static int dos_shares(int64_t n_freq)
+{
+    return (int)std::max<int64_t>(1, SqwTiles<R>::NT / n_freq);
+}
+
+// rows of part a launch over `groups` column groups writes
+template <typename R> int64_t dos_fused_rows(int64_t groups, int64_t n_freq)
+{
+    int dev = 0, ncu = 0;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
+    // two workgroups per CU by the LDS of their tiles
+    return std::min<int64_t>(groups, 2 * std::max(1, ncu)) * dos_shares<R>(n_freq);
+}
+
+template <typename R> bool dos_fused_ok(int64_t n_freq) { return n_freq <= (int64_t)DOS_ACC * SqwTiles<R>::NT; }
+
 template <typename R>
 void launch_dos_fused(const DosParams &p, const RadixPlan &rp, int cols, const float *vel, const int *at_ind,
                       const typename cplx<R>::T *tw, const double *win, double *part, hipStream_t st)
 {
     constexpr int E = SqwTiles<R>::E, NT = SqwTiles<R>::NT;
-    const unsigned nb = (unsigned)((p.nc + cols - 1) / cols);
+    const int64_t ng = (p.nc + cols - 1) / cols;
+    const int nh = dos_shares<R>(p.n_freq);
     // set once per process (a function-local static initialises thread-safely)
     static const bool attr = [] {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_dos_fused<R, E, NT>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)SQW_MAX_LDS);
+        for (const void *fn : {reinterpret_cast<const void *>(&k_dos_fused<R, E, NT, 1>),
+                               reinterpret_cast<const void *>(&k_dos_fused<R, E, NT, DOS_ACC>)})
+            (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SQW_MAX_LDS);
         return true;
     }();
     (void)attr;
-    hipLaunchKernelGGL((k_dos_fused<R, E, NT>), dim3(nb), dim3(NT), dos_fused_lds<R>(p.T, cols), st, p, rp, cols,
-                       make_fdiv((uint32_t)cols), reinterpret_cast<const float2 *>(vel),
-                       reinterpret_cast<const int4 *>(at_ind), tw, win, part);
+    const dim3 grid((unsigned)(dos_fused_rows<R>(ng, p.n_freq) / nh));
+    const size_t lds = dos_fused_lds<R>(p.T, cols);
+    const FDiv dc = make_fdiv((uint32_t)cols), df = make_fdiv((uint32_t)p.n_freq);
+    const float2 *v = reinterpret_cast<const float2 *>(vel);
+    const int4 *ind = reinterpret_cast<const int4 *>(at_ind);
+    if (p.n_freq <= NT)
+        hipLaunchKernelGGL((k_dos_fused<R, E, NT, 1>), grid, dim3(NT), lds, st, p, rp, cols, dc, df, nh, (int)ng, v,
+                           ind, tw, win, part);
+    else
+        hipLaunchKernelGGL((k_dos_fused<R, E, NT, DOS_ACC>), grid, dim3(NT), lds, st, p, rp, cols, dc, df, nh, (int)ng,
+                           v, ind, tw, win, part);
 }
 
 // part2[g][i] = sum over the rows r = g * per .. of part[r][i], in order
@@ -914,6 +1020,8 @@ void launch_sqw_single(const SqwParams &p, const RadixPlan &rp, int cols, const 
     template void launch_iqt<R>(const SqwParams &, const cplx<R>::T *, const float *, double *, double *, hipStream_t); \
     template void launch_iqt_fft<R>(const SqwParams &, const RadixPlan &, int, const cplx<R>::T *, const double2 *,  \
                                     const float *, double *, double *, hipStream_t);                                 \
+    template int64_t dos_fused_rows<R>(int64_t, int64_t);                                                             \
+    template bool dos_fused_ok<R>(int64_t);                                                                           \
     template size_t dos_fused_lds<R>(int64_t, int);                                                                   \
     template void launch_dos_fused<R>(const DosParams &, const RadixPlan &, int, const float *, const int *,          \
                                       const cplx<R>::T *, const double *, double *, hipStream_t);
