@@ -24,6 +24,7 @@ struct Geo {
     int BY, BZ;       // sort-bin extent along y, z
     int nbY, nbZ;     // number of sort bins along y, z
     int nbins;
+    int BR;           // sort bins (along y) per bin of the covering bound
 };
 
 // Sorted point record: first kernel cell (wrapped) and offset of the point
@@ -62,6 +63,7 @@ struct TransformInfo {
     int64_t bs0;      // first entry of the transform's binstart block (nbins + 1 entries)
     int nch, nbins;
     int sxsh, nseg;   // x segments of the covering bound: 2^sxsh cells (>= w), nseg of them
+    int br;            // sort bins per bin of the covering bound (consecutive ones)
 };
 
 struct ColPass {
@@ -216,7 +218,7 @@ template <typename R> size_t spread_lds_twiddles(int by, int bz, int n1, int w, 
 // so rows come in pairs) and the FP32 narrow kernel's dynamic LDS
 template <typename R> bool spread_real_ok(int rows);
 size_t spread_lds_real(int rows, int n1, int w);
-// binmax[bs0 + b] = largest number of bin b's points whose first kernel cell
+// binmax[bs0 + b] = largest number of bound bin b's points whose first kernel cell
 // lies in 3 cyclically consecutive x segments (a bound on how many of them
 // cover any one cell of a row)
 template <typename R>

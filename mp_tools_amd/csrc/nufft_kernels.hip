@@ -451,34 +451,38 @@ __global__ void k_binstart(const int64_t *__restrict__ Hs, const TransformInfo *
     binstart[ti.bs0 + b] = (b < ti.nbins && ti.nch > 0) ? Hs[ti.hbase + (int64_t)b * ti.nch] : ti.p1;
 }
 
-// Covering bound of the FP32 spread (one wave per bin): a cell x of a row is
-// covered by the points whose first kernel cell lies in [x - w + 1, x]
-// (cyclically), a window of w <= 2^sxsh cells that meets at most 3
-// cyclically consecutive segments of 2^sxsh cells (the last segment may be
-// short).  The largest count over such segment triples bounds the number of
-// the bin's points covering any cell.
-template <typename R>
+// Covering bound of the FP32 spread, per bound bin (br sort bins; W waves per
+// bin): a cell x of a row is covered by the points whose first kernel cell
+// lies in [x - w + 1, x] (cyclically), a window of w <= 2^sxsh cells that
+// meets at most 3 cyclically consecutive segments of 2^sxsh cells (the last
+// segment may be short).  The largest count over such segment triples bounds
+// the number of the bin's points covering any cell.  Few bins of many points
+// (20 planes of 320 x 320 cells: 400 bins of 8,192 points) take a workgroup
+// per bin: 76 us with a wave each, 20 so.
+template <typename R, int W>
 __global__ void k_binmax(const PtRec<R> *__restrict__ srec, const int64_t *__restrict__ binstart,
                          const TransformInfo *__restrict__ tinfo, int *__restrict__ binmax)
 {
-    __shared__ int hist[4][64];
+    constexpr int NB = W >= 4 ? 1 : 4;  // bins per block
+    __shared__ int hist[NB][64];
     const TransformInfo ti = tinfo[blockIdx.y];
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int b = blockIdx.x * 4 + wv;
-    hist[wv][lane] = 0;
+    const int hb = NB == 1 ? 0 : wv;
+    const int b = blockIdx.x * NB + hb, nb = ti.nbins / ti.br;
+    if (wv < NB) hist[wv][lane] = 0;
     __syncthreads();
-    if (b < ti.nbins) {
-        const int64_t p0 = binstart[ti.bs0 + b], p1 = binstart[ti.bs0 + b + 1];
-        for (int64_t p = p0 + lane; p < p1; p += 64) {
+    if (b < nb) {
+        const int64_t p0 = binstart[ti.bs0 + (int64_t)b * ti.br], p1 = binstart[ti.bs0 + (int64_t)(b + 1) * ti.br];
+        for (int64_t p = p0 + (NB == 1 ? (int)threadIdx.x : lane); p < p1; p += 64 * W) {
             const int sg = min(max(srec[p].lx, 0) >> ti.sxsh, ti.nseg - 1);
-            atomicAdd(&hist[wv][sg], 1);
+            atomicAdd(&hist[hb][sg], 1);
         }
     }
     __syncthreads();
-    if (b < ti.nbins) {
+    if (b < nb && wv < NB) {
         const int ns = ti.nseg;
         int v = 0;
-        if (lane < ns) v = hist[wv][lane] + hist[wv][(lane + ns - 1) % ns] + hist[wv][(lane + ns - 2) % ns];
+        if (lane < ns) v = hist[hb][lane] + hist[hb][(lane + ns - 1) % ns] + hist[hb][(lane + ns - 2) % ns];
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
         if (lane == 0) binmax[ti.bs0 + b] = v;
@@ -756,8 +760,12 @@ void launch_binmax(const PtRec<R> *srec, const int64_t *binstart, const Transfor
                    int *binmax, hipStream_t st)
 {
     if (ntr <= 0 || max_nbins <= 0) return;
-    hipLaunchKernelGGL((k_binmax<R>), dim3((unsigned)((max_nbins + 3) / 4), (unsigned)ntr), dim3(256), 0, st, srec,
-                       binstart, tinfo, binmax);
+    if ((int64_t)max_nbins * ntr < 4096)  // fewer waves than the chip holds with one per bin
+        hipLaunchKernelGGL((k_binmax<R, 16>), dim3((unsigned)max_nbins, (unsigned)ntr), dim3(1024), 0, st, srec,
+                           binstart, tinfo, binmax);
+    else
+        hipLaunchKernelGGL((k_binmax<R, 1>), dim3((unsigned)((max_nbins + 3) / 4), (unsigned)ntr), dim3(256), 0, st,
+                           srec, binstart, tinfo, binmax);
 }
 
 template <typename R>

@@ -507,11 +507,17 @@ __device__ __forceinline__ void runs_publish(RunTable &S, int pb, const SpreadJo
     int cb = 0x7fffffff;
     if (bound && J.binmax) {
         const int *bm = J.binmax + (int64_t)t * J.bin_tstride * (g.nbins + 1);
-        const int nv = nyb * nzb;
+        // over the bound's bins, BR sort bins each
+        Geo gb = g;
+        gb.BY = g.BY * g.BR;
+        gb.nbY = g.nbY / g.BR;
+        int yb, ny, zb, nz;
+        rect_bins(gb, y0, z0, by, bz, yb, ny, zb, nz);
+        const int nv = ny * nz;
         int sum = 0;
         for (int i = lane; i < nv; i += 64) {
-            const int k = i / nyb, jy = i - k * nyb;
-            sum += gload(bm + posmod(zlo + k, g.nbZ) * g.nbY + posmod(ylo + jy, g.nbY));
+            const int k = i / ny, jy = i - k * ny;
+            sum += gload(bm + posmod(zb + k, gb.nbZ) * gb.nbY + posmod(yb + jy, gb.nbY));
         }
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
