@@ -585,25 +585,30 @@ __global__ __launch_bounds__(NT) void k_colfft(const ColJob<R> *__restrict__ job
     // kh) goes to its place and, when k1 < 0, its mirror (2 h - kk, 2 h2 - km,
     // 2 h1 - kh), where in range, as the conjugate: every mode of the map is
     // written once.
+    // (the job's fields in registers: read through J after each store they
+    // would be loaded again)
+    const bool herm = FINAL && cp.herm, cj = cp.conj != 0, mid = cp.hmid != 0;
+    const int N1 = cp.hN1, h1 = N1 / 2, N2 = cp.hN2, h2 = N2 / 2, H1 = cp.hH1, H1v = cp.hH1v;
+    const int64_t hsa = cp.hsa;
+    const FDiv dH1 = cp.dH1;
+    CS *const map = J.out + (FINAL ? (int64_t)grp * cp.out_tstride + (herm ? 0 : (int64_t)o * N * inner + col0) : 0);
     auto emit = [&](int kk, int c, CS x) {
-        if (cp.conj) x.y = -x.y;
-        CS *dst = J.out + (int64_t)grp * cp.out_tstride;
-        if (!cp.herm) {
-            if (kk < N) dst[(int64_t)o * N * inner + col0 + (int64_t)kk * inner + c] = x;
+        if (cj) x.y = -x.y;
+        if (!herm) {
+            if (kk < N) map[(int64_t)kk * inner + c] = x;
             return;
         }
-        const int N1 = cp.hN1, h1 = N1 / 2, N2 = cp.hN2, h2 = N2 / 2;
         const int col = col0 + c;
         int km = 0, kh = col;
-        if (cp.hmid) {
-            km = (int)fdiv((uint32_t)col, cp.dH1);
-            kh = col - km * cp.hH1;
+        if (mid) {
+            km = (int)fdiv((uint32_t)col, dH1);
+            kh = col - km * H1;
         }
-        if (kh >= cp.hH1v) return;  // pad column
-        if (kk < N && km < N2) dst[(int64_t)kk * cp.hsa + (int64_t)km * N1 + kh] = x;
-        const int ka = 2 * h - kk, kmm = cp.hmid ? 2 * h2 - km : 0, kx = 2 * h1 - kh;
+        if (kh >= H1v) return;  // pad column
+        if (kk < N && km < N2) map[(int64_t)kk * hsa + (int64_t)km * N1 + kh] = x;
+        const int ka = 2 * h - kk, kmm = mid ? 2 * h2 - km : 0, kx = 2 * h1 - kh;
         if (kh < h1 && kx < N1 && ka >= 0 && ka < N && kmm >= 0 && kmm < N2)
-            dst[(int64_t)ka * cp.hsa + (int64_t)kmm * N1 + kx] = cmk<CS>(x.x, -x.y);
+            map[(int64_t)ka * hsa + (int64_t)kmm * N1 + kx] = cmk<CS>(x.x, -x.y);
     };
     for (int s = 0; s < nsp; ++s) {
         const int t = FINAL ? grp * cp.nsp + s : grp;
@@ -646,14 +651,19 @@ __global__ __launch_bounds__(NT) void k_colfft(const ColJob<R> *__restrict__ job
                 dst[(int64_t)kk * inner + c] = cmk<CS>((R)x.x, (R)x.y);
             }
         } else {
+            const R *phinv = J.phinv;
+            const float *wtab = J.wtab;
+            const R ws = J.wsc ? J.wsc[s] : (R)1;
+            const int64_t NQ = cp.NQ;
+            const FDiv dcols = cp.dcols;
             for (int i = threadIdx.x; i < NO * cols; i += NT) {
-                const int kk = (int)fdiv((uint32_t)i, cp.dcols), c = i - kk * cols;
+                const int kk = (int)fdiv((uint32_t)i, dcols), c = i - kk * cols;
                 int f = kk - h;
                 if (f < 0) f += n;
-                R wv = J.phinv[phi_ix(kk)];
+                R wv = phinv[phi_ix(kk)];
                 // (a half-spectrum pass has no per-Q table: the host keeps those jobs full)
-                if (J.wtab) wv *= (c < ncol) ? (R)J.wtab[(int64_t)s * cp.NQ + (int64_t)kk * inner + col0 + c] : (R)0;
-                else if (J.wsc) wv *= J.wsc[s];
+                if (wtab) wv *= (c < ncol) ? (R)wtab[(int64_t)s * NQ + (int64_t)kk * inner + col0 + c] : (R)0;
+                else wv *= ws;
                 C x = cscale(tile[f * cols + c], wv);
                 if (s > 0) x = cadd(acc[i], x);
                 if (s + 1 < nsp) acc[i] = x;
