@@ -80,6 +80,10 @@ int mpsq_get_sort_perm(mpsq_plan plan, int32_t *perm);
  * out[0..2] = n1,n2,n3, out[3] = w, out[4] = by, out[5] = bz, out[6] = BY,
  * out[7] = BZ. */
 int mpsq_plan_info(mpsq_plan plan, int64_t *out);
+/* The stream the plan's work is queued on (a hipStream_t; the caller's, or
+ * the plan's own, which lives until mpsq_destroy): for a caller that orders
+ * its own work or the reuse of its memory after mpsq_execute_dev. */
+void *mpsq_plan_stream(mpsq_plan plan);
 
 /* ---------------- FINUFFT-shaped plan API, FP32 ---------------- */
 typedef struct mpsq_planf_s *mpsq_planf;
@@ -92,6 +96,7 @@ int mpsqf_execute_dev(mpsq_planf plan, const float *d_c, float *d_f);
 int mpsqf_destroy(mpsq_planf plan);
 int mpsqf_get_sort_perm(mpsq_planf plan, int32_t *perm);
 int mpsqf_plan_info(mpsq_planf plan, int64_t *out);
+void *mpsqf_plan_stream(mpsq_planf plan);
 
 /* ---------------- simple interface (FINUFFT's finufft{1,2,3}d1) ---------------- */
 int mpsq_nufft1d1(int64_t nj, const double *xj, const double *cj, int iflag, double eps, int64_t ms,

@@ -27,9 +27,9 @@ FP64 = 1
 # every symbol include/mpsq.h declares
 EXPORTS = [
     "mpsq_default_opts", "mpsq_makeplan", "mpsq_setpts", "mpsq_execute", "mpsq_setpts_dev",
-    "mpsq_execute_dev", "mpsq_destroy", "mpsq_get_sort_perm", "mpsq_plan_info",
+    "mpsq_execute_dev", "mpsq_destroy", "mpsq_get_sort_perm", "mpsq_plan_info", "mpsq_plan_stream",
     "mpsqf_makeplan", "mpsqf_setpts", "mpsqf_execute", "mpsqf_setpts_dev", "mpsqf_execute_dev",
-    "mpsqf_destroy", "mpsqf_get_sort_perm", "mpsqf_plan_info",
+    "mpsqf_destroy", "mpsqf_get_sort_perm", "mpsqf_plan_info", "mpsqf_plan_stream",
     "mpsq_nufft1d1", "mpsq_nufft2d1", "mpsq_nufft3d1",
     "finufft1d1_", "finufft2d1_", "finufft3d1_",
     "mpsq_makeplan_", "mpsq_setpts_", "mpsq_execute_", "mpsq_destroy_",
@@ -137,6 +137,8 @@ def load():
         getattr(L, f"{pre}_destroy").argtypes = [vp]
         getattr(L, f"{pre}_get_sort_perm").argtypes = [vp, vp]
         getattr(L, f"{pre}_plan_info").argtypes = [vp, vp]
+        getattr(L, f"{pre}_plan_stream").argtypes = [vp]
+        getattr(L, f"{pre}_plan_stream").restype = vp
     L.mpsq_nufft1d1.argtypes = [i64, vp, vp, i32, dbl, i64, vp, vp]
     L.mpsq_nufft2d1.argtypes = [i64, vp, vp, vp, i32, dbl, i64, i64, vp, vp]
     L.mpsq_nufft3d1.argtypes = [i64, vp, vp, vp, vp, i32, dbl, i64, i64, i64, vp, vp]

@@ -2450,6 +2450,8 @@ int mpsq_destroy(mpsq_plan p)
 int mpsq_get_sort_perm(mpsq_plan p, int32_t *perm) { return perm_impl<double>(reinterpret_cast<Plan<double> *>(p), perm); }
 int mpsq_plan_info(mpsq_plan p, int64_t *out) { return info_impl<double>(reinterpret_cast<Plan<double> *>(p), out); }
 
+void *mpsq_plan_stream(mpsq_plan p) { return p ? reinterpret_cast<Plan<double> *>(p)->core.st : nullptr; }
+
 // ---- FP32 plan ----
 int mpsqf_makeplan(int type, int dim, const int64_t *n_modes, int iflag, int ntrans, double eps, mpsq_planf *plan,
                    const mpsq_opts *opts)
@@ -2484,6 +2486,8 @@ int mpsqf_destroy(mpsq_planf p)
 }
 int mpsqf_get_sort_perm(mpsq_planf p, int32_t *perm) { return perm_impl<float>(reinterpret_cast<Plan<float> *>(p), perm); }
 int mpsqf_plan_info(mpsq_planf p, int64_t *out) { return info_impl<float>(reinterpret_cast<Plan<float> *>(p), out); }
+
+void *mpsqf_plan_stream(mpsq_planf p) { return p ? reinterpret_cast<Plan<float> *>(p)->core.st : nullptr; }
 
 // ---- simple interface with a one-entry plan cache ----
 // The reference calls the simple interface once per frame and species from

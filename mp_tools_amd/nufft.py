@@ -20,6 +20,7 @@ torch stream that was current when the plan was made).
 from __future__ import annotations
 
 import ctypes as C
+from collections import deque
 
 import numpy as np
 
@@ -68,7 +69,9 @@ class Plan:
         self._h = h
         self.M = None
         self._keep = None
-        self._inflight = None
+        self._device = int(device)
+        self._stream = int(stream or 0)  # 0: a stream of the plan's own
+        self._inflight = deque()
 
     # -- points -------------------------------------------------------------
     def setpts(self, x, y=None, z=None):
@@ -88,6 +91,7 @@ class Plan:
             ptrs = [v.ctypes.data for v in co] + [None] * (3 - self.dim)
             rc = getattr(self._L, f"{self._pre}_setpts")(self._h, M, *ptrs)
         _lib.check("setpts", rc)
+        self._inflight.clear()  # the call waited for the plan's stream
         self._keep = co
         self.M = M
         return rc
@@ -108,11 +112,9 @@ class Plan:
                 raise ValueError("strength count does not match M * n_trans")
             if out is None:
                 out = torch.empty(self._out_shape(), dtype=tdt, device=c.device)
+            self._release()
             rc = getattr(self._L, f"{self._pre}_execute_dev")(self._h, c.data_ptr(), out.data_ptr())
-            # the call returns with its work queued on the plan's stream, which
-            # torch's allocator does not know: held until the plan's next call,
-            # so that their memory does not go to another plan's work meanwhile
-            self._inflight = (c, out)
+            self._hold((c, out))
         else:
             c = np.ascontiguousarray(data, dtype=self.dtype).ravel()
             if c.size != self.M * self.n_trans:
@@ -122,6 +124,40 @@ class Plan:
             rc = getattr(self._L, f"{self._pre}_execute")(self._h, c.ctypes.data, out.ctypes.data)
         _lib.check("execute", rc)
         return out
+
+    # -- tensors of queued calls ----------------------------------------------
+    # A device execute returns with its work queued on the plan's stream.  Where
+    # that is not the torch stream its tensors were allocated on, torch's
+    # allocator would hand their memory to the next plan's tensors once the
+    # caller drops them, while the work still runs.  They are held until the
+    # work is done, whatever number of calls later that is: [event, tensors] per
+    # call, the event recorded before the next call's work is queued (a plan that
+    # alternates setpts, which waits, and execute records none).  At most HOLD
+    # earlier calls are held: the host waits for the oldest before it queues more.
+    HOLD = 2
+
+    def _mark(self):
+        """An event behind all work queued on the plan's stream."""
+        import torch
+        ev = torch.cuda.Event()
+        ev.record(torch.cuda.ExternalStream(getattr(self._L, f"{self._pre}_plan_stream")(self._h), device=self._device))
+        return ev
+
+    def _release(self):
+        """Drop what finished calls held, before another one is queued."""
+        q = self._inflight
+        if q and q[-1][0] is None:
+            q[-1][0] = self._mark()
+        while q and (q[0][0].query() or len(q) > self.HOLD):
+            q[0][0].synchronize()
+            q.popleft()
+
+    def _hold(self, tensors):
+        if self._stream:
+            import torch
+            if torch.cuda.current_stream(self._device).cuda_stream == self._stream:
+                return  # the allocator orders reuse on this stream itself
+        self._inflight.append([None, tensors])
 
     def sort_perm(self) -> np.ndarray:
         """Bin-sort permutation of the last setpts (perm[k] = input index)."""
@@ -139,7 +175,7 @@ class Plan:
         if getattr(self, "_h", None) and self._h.value:
             getattr(self._L, f"{self._pre}_destroy")(self._h)  # waits for the plan's work
             self._h = C.c_void_p()
-            self._inflight = None
+            self._inflight.clear()
 
     def __del__(self):
         try:
