@@ -92,7 +92,7 @@ def make_spec(dim, n_modes, species_counts, eps=1e-6, precision="fp32", iflag=-1
     s.opts.tile_by, s.opts.tile_bz = int(tile_by), int(tile_bz)
     info = dict(dim=dim, n_modes=n_modes, NQ=NQ, precision=precision, fp64=fp64,
                 cdtype=torch.complex128 if fp64 else torch.complex64, nsp=nsp, n_tot=n_tot,
-                combine=bool(combine),
+                combine=bool(combine), device=int(device),
                 Mact=int(counts.sum() if mask is None else counts[np.asarray(mask) != 0].sum()))
     return s, keep, info
 
@@ -205,8 +205,11 @@ class SqwEngine:
 
     def set_workspace(self, buf, frames=1):
         """Keep the intermediate grids of runs of up to ``frames`` frames in
-        the CUDA tensor ``buf`` (held until another is set; None: memory of
-        the engine's own)."""
+        the CUDA tensor ``buf`` (contiguous, on the engine's device, at least
+        ``workspace_bytes(frames)`` bytes from a multiple of 256; held until
+        another is set; None: memory of the engine's own)."""
+        if buf is not None and not (buf.is_cuda and buf.device.index == self.device and buf.is_contiguous()):
+            raise ValueError(f"the workspace must be a contiguous tensor on cuda:{self.device}")
         n = 0 if buf is None else buf.numel() * buf.element_size()
         _lib.check("sqw_set_workspace", self._L.mpsq_sqw_set_workspace(self._h, None if buf is None else buf.data_ptr(),
                                                                       n, int(frames)))
@@ -231,8 +234,9 @@ class SqwEngine:
 
     def destroy(self):
         if getattr(self, "_h", None) and self._h.value:
-            self._L.mpsq_sqw_destroy(self._h)
+            self._L.mpsq_sqw_destroy(self._h)  # waits for the engine's work
             self._h = C.c_void_p()
+            self._ws = None
 
     def __del__(self):
         try:
