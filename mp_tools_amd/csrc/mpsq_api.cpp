@@ -489,13 +489,7 @@ template <typename R> struct Core {
         // by + w <= n2 and bz + w <= n3 keep the rows a kernel stencil has in
         // one tile contiguous
         real = real_;
-        // real strengths: up to 32 rows where the complex kernel's registers
-        // stop short of that (n1 = 512: 16 -> 32); grids that already allow
-        // 32 rows or more keep their cap, since taller tiles of dense inputs
-        // overflow the narrow kernel's covering bound and every wide pass
-        // re-walks the whole tile's candidates
-        rows_max = spread_max_rows<R>((int)n[0]);
-        if (real && rows_max < 32) rows_max = std::min(2 * rows_max, 32);
+        rows_max = real ? spread_max_rows_real<R>((int)n[0]) : spread_max_rows<R>((int)n[0]);
         // FP64 tiles of real strengths: no more rows than let two workgroups
         // share a CU (fine rows of 1024 cells: 4 rows, 51 KB, instead of 8,
         // 86 KB; 30,000 points 0.124 -> 0.113 ms, 3 million 1.62 -> 1.49)
@@ -539,9 +533,10 @@ template <typename R> struct Core {
         }
         if (o->tile_by > 0 && dim >= 2 && n[1] % o->tile_by == 0) by = o->tile_by;
         if (o->tile_bz > 0 && dim >= 3 && n[2] % o->tile_bz == 0) bz = o->tile_bz;
-        if (by * bz > rows_max || by > bmax || bz > bmax) throw Err{MPSQ_ERR_BAD_ARG};
-        if (spread_lds<R>(by, bz, (int)n[0], w, real) > 156 * 1024 ||
-            (real && sizeof(R) == 4 && spread_lds_real(by * bz, (int)n[0], w) > 156 * 1024))
+        if (!spread_tile_ok<R>(by, bz, (int)n[0], real)) throw Err{MPSQ_ERR_BAD_ARG};
+        const bool rk = real && spread_real_ok<R>(by * bz);  // (as real_launch)
+        if (spread_lds<R>(by, bz, (int)n[0], w, rk) > 156 * 1024 ||
+            (rk && sizeof(R) == 4 && spread_lds_real(by * bz, (int)n[0], w) > 156 * 1024))
             throw Err{MPSQ_ERR_SIZE};
         if ((dim >= 2 && by + w > n[1]) || (dim >= 3 && bz + w > n[2])) throw Err{MPSQ_ERR_BAD_ARG};
         g.by = by;

@@ -207,6 +207,9 @@ int spread_max_tile_b();
 int spread_max_wide_passes();
 // largest tile (rows of the whole x extent) of a fine grid of n1 cells in x
 template <typename R> int spread_max_rows(int n1);
+template <typename R> int spread_max_rows_real(int n1);  // of real strengths
+// whether the kernels take a by x bz tile
+template <typename R> bool spread_tile_ok(int by, int bz, int n1, bool real);
 // and the rows of one wide pass of a by x bz tile (real: of real strengths)
 template <typename R> int spread_group_rows(int by, int bz, int n1, bool real);
 // dynamic LDS of the launches of complex strengths, or (real) of the wide

@@ -72,7 +72,7 @@ template <> struct SpreadCfg<double> { static constexpr int E = 8, NT = 512; };
 struct NarrowCfg {
     static constexpr int E = 8, NT = 512;
 };
-constexpr int MAX_WIDE_PASSES = 16;  // wide passes of a tile (a tile has at most twice the rows one pass holds)
+constexpr int MAX_WIDE_PASSES = 16;  // wide passes of a queued tile (spread_tile_ok; shapes up to 16 x 16 take at most 15)
 
 constexpr int MAX_TILE_B = 16;   // by, bz <= 16
 constexpr int NARROW_MAX = 256;  // largest covering bound of a 32-bit (narrow) FP32 tile
@@ -200,6 +200,31 @@ template <typename R> int spread_group_rows(int by, int bz, int n1, bool real)
         if (by % k == 0 && fits(k)) return k;
     return 1;
 }
+// Rows of the largest tile of real strengths: twice the complex kernel's where
+// that has fewer than 32 (n1 = 512: 16 -> 32).  Grids that already allow 32
+// rows or more keep their cap, since taller tiles of dense inputs overflow the
+// narrow kernel's covering bound.
+template <typename R> int spread_max_rows_real(int n1)
+{
+    const int m = spread_max_rows<R>(n1);
+    return m < 32 ? std::min(2 * m, 32) : m;
+}
+// rows pair up (the real narrow kernel)
+__host__ __device__ inline bool spread_real_fits(int rows) { return rows >= 2 && rows % 2 == 0; }
+// whether a tile of real strengths takes the real kernels
+template <typename R> bool spread_real_ok(int rows) { return sizeof(R) == 8 || spread_real_fits(rows); }
+// Whether the kernels take a by x bz tile: its rows fit the x FFT of the
+// narrow kernel it runs on (a tile of real strengths whose rows do not pair
+// up runs on the complex one), a queued FP32 tile's wide passes fit its
+// entries of the queue, and an FP64 tile is one pass.
+template <typename R> bool spread_tile_ok(int by, int bz, int n1, bool real)
+{
+    const int rows = by * bz;
+    if (by < 1 || bz < 1 || by > MAX_TILE_B || bz > MAX_TILE_B) return false;
+    const bool rk = real && spread_real_ok<R>(rows);
+    if (rows > (rk ? spread_max_rows_real<R>(n1) : spread_max_rows<R>(n1))) return false;
+    return rows / spread_group_rows<R>(by, bz, n1, rk) <= (sizeof(R) == 4 ? MAX_WIDE_PASSES : 1);
+}
 // bytes of the tile region (accumulators / FFT rows); the twiddles follow it
 __host__ __device__ constexpr int narrow_bias(int w) { return (8 * w + 15) / 16 * 16; }
 template <typename R> size_t spread_tile_bytes(int by, int bz, int n1, int w, bool real)
@@ -233,8 +258,6 @@ __host__ __device__ inline int spread_real_tw_offset(int rows, int n1, int w)
 {
     return (narrow_bias(w) + rows * spread_row_stride_x(n1, w) * 4 + 15) / 16 * 16;
 }
-// rows pair up
-__host__ __device__ inline bool spread_real_fits(int rows) { return rows >= 2 && rows % 2 == 0; }
 // each wave can transform its own pairs: they fit its lanes' registers
 // (2E elements per lane) and a pair's accumulators end inside its FFT slot
 // (else the block-wide FFT)

@@ -26,7 +26,6 @@ size_t spread_lds_real(int rows, int n1, int w)
 {
     return (size_t)spread_real_tw_offset(rows, n1, w) + (size_t)n1 * 8 + (size_t)(n1 / 2) * 4 + (size_t)rows * 8;
 }
-template <typename R> bool spread_real_ok(int rows) { return sizeof(R) == 8 || spread_real_fits(rows); }
 template <typename R> int spread_tile_elems() { return SpreadCfg<R>::E * SpreadCfg<R>::NT; }
 int spread_max_runs() { return MAX_RUNS; }
 int spread_max_tile_b() { return MAX_TILE_B; }
@@ -82,6 +81,8 @@ void launch_spread_jobs(const SpreadJob<R> *jobs, const int *tile0s, int njobs, 
 #define MPSQ_SPREAD_INST(R)                                                                                           \
     template bool spread_real_ok<R>(int);                                                                             \
     template int spread_tile_elems<R>();                                                                              \
+    template int spread_max_rows_real<R>(int);                                                                        \
+    template bool spread_tile_ok<R>(int, int, int, bool);                                                             \
     template int spread_max_rows<R>(int);                                                                             \
     template int spread_group_rows<R>(int, int, int, bool);                                                           \
     template size_t spread_lds<R>(int, int, int, int, bool);                                                          \
