@@ -20,18 +20,9 @@
 
 #include "mpsq.h"
 #include "mpsq_kernels.h"
+#include "mpsq_buffers.h"
 
 namespace mpsq {
-
-struct Err {
-    int code;
-};
-
-#define HIPCHK(x)                                                                                                     \
-    do {                                                                                                              \
-        hipError_t e_ = (x);                                                                                          \
-        if (e_ != hipSuccess) throw Err{MPSQ_ERR_DEVICE};                                                             \
-    } while (0)
 
 // Error flags the kernels raise in a device int: bit 0 a non-finite point
 // coordinate, bit 1 an internal bound check of the spread (a candidate run
@@ -41,40 +32,6 @@ static void throw_bad(int hbad)
     if (hbad & 2) throw Err{MPSQ_ERR_DEVICE};
     if (hbad & 1) throw Err{MPSQ_ERR_NONFINITE_POINT};
 }
-
-struct DevBuf {
-    void *p = nullptr;
-    size_t bytes = 0;
-    bool lent = false;  // the memory is the caller's
-    // use the caller's memory (which outlives the buffer's use of it)
-    void adopt(void *q, size_t b)
-    {
-        release();
-        p = q;
-        bytes = b;
-        lent = true;
-    }
-    void ensure(size_t b)
-    {
-        if (b <= bytes && p) return;
-        release();
-        if (b == 0) return;
-        if (hipMalloc(&p, b) != hipSuccess) {
-            p = nullptr;
-            throw Err{MPSQ_ERR_DEVICE};
-        }
-        bytes = b;
-    }
-    void release()
-    {
-        if (p && !lent) (void)hipFree(p);
-        p = nullptr;
-        bytes = 0;
-        lent = false;
-    }
-    template <typename T> T *as() const { return static_cast<T *>(p); }
-    ~DevBuf() { release(); }
-};
 
 // ---------------------------------------------------------------------------
 // kernel parameters and fine grid
@@ -289,83 +246,6 @@ struct StageTimer {
 };
 
 enum { ST_STAGE = 0, ST_SORT = 1, ST_SPREAD = 2, ST_COLPASS = 3, ST_FINAL = 4, ST_REDUCE = 5 };
-
-// ---------------------------------------------------------------------------
-// Job tables: built in pinned host memory and uploaded with one copy per
-// run, ahead of the kernels that read them (stream order).  Before the host
-// rewrites the tables it waits for the previous upload, which keeps a
-// pending copy from reading half-written tables.
-// ---------------------------------------------------------------------------
-struct Arena {
-    unsigned char *h = nullptr;
-    size_t cap = 0, used = 0;
-    DevBuf d;
-    hipEvent_t ev = nullptr;
-    bool pending = false;
-    // what the device has: the first `sent` bytes, uploaded on sent_st; tables
-    // equal to it (a plan's next points, an engine's next batch of frames) are
-    // not uploaded again
-    size_t sent = 0;
-    hipStream_t sent_st = nullptr;
-    bool dirty = true;
-    void begin()
-    {
-        used = 0;
-        dirty = sent == 0;
-    }
-    void touch()
-    {
-        if (pending) HIPCHK(hipEventSynchronize(ev));
-        pending = false;
-        dirty = true;
-    }
-    size_t put_raw(const void *src, size_t bytes)
-    {
-        const size_t off = (used + 255) & ~(size_t)255;
-        if (off + bytes > cap) {
-            size_t nc = std::max<size_t>(cap * 2, 1 << 16);
-            while (nc < off + bytes) nc *= 2;
-            touch();
-            unsigned char *nh = nullptr;
-            HIPCHK(hipHostMalloc(reinterpret_cast<void **>(&nh), nc, hipHostMallocDefault));
-            if (h) {
-                std::memcpy(nh, h, used);
-                (void)hipHostFree(h);
-            }
-            h = nh;
-            cap = nc;
-        }
-        if (bytes && (dirty || off + bytes > sent || std::memcmp(h + off, src, bytes) != 0)) {
-            if (!dirty || pending) touch();
-            std::memcpy(h + off, src, bytes);
-        }
-        used = off + bytes;
-        return off;
-    }
-    template <typename T> size_t put(const std::vector<T> &v) { return put_raw(v.data(), sizeof(T) * v.size()); }
-    void upload(hipStream_t st)
-    {
-        if (used == 0 || (!dirty && used <= sent && st == sent_st)) return;
-        sent = 0;
-        d.ensure(used);
-        if (!ev) HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-        HIPCHK(hipMemcpyAsync(d.p, h, used, hipMemcpyHostToDevice, st));
-        HIPCHK(hipEventRecord(ev, st));
-        pending = true;
-        sent = used;
-        sent_st = st;
-    }
-    template <typename T> const T *dev(size_t off) const
-    {
-        return reinterpret_cast<const T *>(static_cast<const unsigned char *>(d.p) + off);
-    }
-    ~Arena()
-    {
-        if (pending && ev) (void)hipEventSynchronize(ev);
-        if (ev) (void)hipEventDestroy(ev);
-        if (h) (void)hipHostFree(h);
-    }
-};
 
 // Cut the tile-id space [0, cost.size()) into 8 contiguous ranges of about
 // equal total cost, one per XCD.
@@ -1842,7 +1722,7 @@ template <typename R> struct Batch {
         if (use_graph && key == gkey && !gexec) {
             // capture: everything is allocated and the tables are current
             HIPCHK(hipStreamSynchronize(st));
-            for (Arena *a : arenas) a->touch();  // nothing pending may be waited on inside the capture
+            for (Arena *a : arenas) a->settle();  // nothing pending may be waited on inside the capture
             HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
             enqueue(d_pos, T, d_amp, r, d_S, d_Stot, nullptr);
             hipGraph_t g = nullptr;
