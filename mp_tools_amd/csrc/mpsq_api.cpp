@@ -171,14 +171,18 @@ template <typename R> using Cx = typename cplx<R>::T;
 constexpr int IQT_FFT_MIN_LAGS = 16;
 constexpr size_t IQT_FFT_LDS_TARGET = 76 * 1024;
 
+template <typename R> static void fill_twiddles(Cx<R> *tw, int n)
+{
+    for (int m = 0; m < n; ++m) {
+        const double a = -2.0 * M_PI * (double)m / (double)n;
+        tw[m].x = (R)std::cos(a);
+        tw[m].y = (R)std::sin(a);
+    }
+}
 template <typename R> static void upload_twiddles(DevBuf &buf, int n, hipStream_t st, std::vector<Cx<R>> &host)
 {
     host.resize((size_t)n);
-    for (int m = 0; m < n; ++m) {
-        const double a = -2.0 * M_PI * (double)m / (double)n;
-        host[(size_t)m].x = (R)std::cos(a);
-        host[(size_t)m].y = (R)std::sin(a);
-    }
+    fill_twiddles<R>(host.data(), n);
     buf.ensure(sizeof(Cx<R>) * (size_t)n);
     HIPCHK(hipMemcpyAsync(buf.p, host.data(), sizeof(Cx<R>) * (size_t)n, hipMemcpyHostToDevice, st));
 }
@@ -933,45 +937,28 @@ template <typename R> struct Engine {
     DevBuf wsc, wtab, at_ind;
     std::vector<double> wsh;        // active species weights (host copy of wsc)
     Workspace<R> ws;                // buffers when run alone
-    // reduction caches
-    DevBuf win_d, twT;
+    // tables of the reductions, kept while the frames and the window stay
     StageTimer tm;
-    std::vector<double> win_h;
-    std::vector<Cx<R>> twT_h;
-    int win_n = -1, win_kind = -1, twT_n = -1;
-    RadixPlan rpT{};
-    DevBuf twI;                     // FP64 twiddles of the I(Q,t) correlation
-    std::vector<Cx<double>> twI_h;
-    int twI_n = -1;
-    RadixPlan rpI{};
-    // tables of the DFT kernels: twiddles of the window length, and the
-    // window's cosines over the frames
-    DevBuf twN, hann;
-    std::vector<Cx<double>> twN_h, hann_h;
-    int twN_n = -1, hann_n = -1, hann_kind = -1;
-    int64_t hann_T = -1;
+    KeyedTable<double> win;         // one window over all frames
+    KeyedTable<Cx<R>> twT;          // twiddles of the time FFT,
+    KeyedTable<Cx<double>> twI;     // of the I(Q,t) correlation,
+    KeyedTable<Cx<double>> twN;     // of the DFT kernels, and
+    KeyedTable<Cx<double>> hann;    // their window's cosines over the frames
 
-    void dft_twiddles(int n, hipStream_t st)
+    const Cx<double> *dft_twiddles(int n, hipStream_t st)
     {
-        if (twN_n == n) return;
-        upload_twiddles<double>(twN, n, st, twN_h);
-        twN_n = n;
+        return twN.get({n, 0, 0}, (size_t)n, st, [&](Cx<double> *h) { fill_twiddles<double>(h, n); });
     }
-    void hann_table(int64_t T, int n, int kind, hipStream_t st)
+    const Cx<double> *hann_table(int64_t T, int n, int kind, hipStream_t st)
     {
-        if (hann_T == T && hann_n == n && hann_kind == kind) return;
-        hann_h.assign((size_t)T + 1, Cx<double>{0.0, 0.0});
-        const int64_t period = kind == 1 ? n + 1 : n - 1;
-        for (int64_t t = -1; t < T && n > 1; ++t) {
-            const double a = 2.0 * M_PI * (double)((t + period) % period) / (double)period;
-            hann_h[(size_t)(t + 1)].x = std::cos(a);
-            hann_h[(size_t)(t + 1)].y = std::sin(a);
-        }
-        hann.ensure(sizeof(Cx<double>) * hann_h.size());
-        HIPCHK(hipMemcpyAsync(hann.p, hann_h.data(), sizeof(Cx<double>) * hann_h.size(), hipMemcpyHostToDevice, st));
-        hann_T = T;
-        hann_n = n;
-        hann_kind = kind;
+        return hann.get({T, n, kind}, (size_t)T + 1, st, [&](Cx<double> *h) {
+            const int64_t period = kind == 1 ? n + 1 : n - 1;
+            for (int64_t t = -1; t < T && n > 1; ++t) {
+                const double a = 2.0 * M_PI * (double)((t + period) % period) / (double)period;
+                h[t + 1].x = std::cos(a);
+                h[t + 1].y = std::sin(a);
+            }
+        });
     }
 
     int64_t nq() const { return core.N[0] * core.N[1] * core.N[2]; }
@@ -1204,18 +1191,14 @@ template <typename R> struct Engine {
                              iqt_fft_lds(T, 1) <= SQW_MAX_LDS && radix_plan((int)T, rp);
             const int ev = tm.begin(ST_REDUCE, st);
             if (fft) {
-                if (twI_n != (int)T) {
-                    upload_twiddles<double>(twI, (int)T, st, twI_h);
-                    twI_n = (int)T;
-                    rpI = rp;
-                }
+                const Cx<double> *tw = twI.get({T, 0, 0}, (size_t)T, st, [&](Cx<double> *h) { fill_twiddles<double>(h, (int)T); });
                 // columns per block: the most that keep two blocks per CU
                 // (or one, for long series)
                 int cols = 1;
                 while (2 * cols * T <= iqt_fft_tile_elems() && 2 * cols <= SQW_MAX_COLS &&
                        iqt_fft_lds(T, 2 * cols) <= IQT_FFT_LDS_TARGET)
                     cols *= 2;
-                launch_iqt_fft<R>(p, rpI, cols, amp, twI.as<Cx<double>>(), r->d_qfac, d_S, d_Stot, st);
+                launch_iqt_fft<R>(p, rp, cols, amp, tw, r->d_qfac, d_S, d_Stot, st);
             } else {
                 launch_iqt<R>(p, amp, r->d_qfac, d_S, d_Stot, st);
             }
@@ -1234,44 +1217,34 @@ template <typename R> struct Engine {
         const bool direct = p.n_f == 0 || T * p.n_f <= 400;
         const bool single = (p.n_frame == 1) && !direct && (T <= sqw_tile_elems<R>()) &&
                             sqw_single_lds<R>(T, 1) <= SQW_MAX_LDS && radix_plan((int)T, rp);
-        if (p.n_frame == 1) {
-            if (win_n != (int)T || win_kind != r->win_kind) {
-                win_h.resize((size_t)T);
+        const double *win_d = nullptr;
+        if (p.n_frame == 1)
+            win_d = win.get({T, r->win_kind, 0}, (size_t)T, st, [&](double *h) {
                 for (int64_t i = 0; i < T; ++i) {
-                    if (T <= 1) win_h[i] = 1.0;
-                    else if (r->win_kind == 0) win_h[i] = 0.5 * (1.0 - std::cos(2.0 * M_PI * (double)i / (double)(T - 1)));
-                    else win_h[i] = 0.5 * (1.0 - std::cos(2.0 * M_PI * (double)(i + 1) / (double)(T + 1)));
+                    if (T <= 1) h[i] = 1.0;
+                    else if (r->win_kind == 0) h[i] = 0.5 * (1.0 - std::cos(2.0 * M_PI * (double)i / (double)(T - 1)));
+                    else h[i] = 0.5 * (1.0 - std::cos(2.0 * M_PI * (double)(i + 1) / (double)(T + 1)));
                 }
-                win_d.ensure(sizeof(double) * (size_t)T);
-                HIPCHK(hipMemcpyAsync(win_d.p, win_h.data(), sizeof(double) * (size_t)T, hipMemcpyHostToDevice, st));
-                win_n = (int)T;
-                win_kind = r->win_kind;
-            }
-        }
+            });
         if (single) {
-            if (twT_n != (int)T) {
-                upload_twiddles<R>(twT, (int)T, st, twT_h);
-                twT_n = (int)T;
-                rpT = rp;
-            }
+            const Cx<R> *tw = twT.get({T, 0, 0}, (size_t)T, st, [&](Cx<R> *h) { fill_twiddles<R>(h, (int)T); });
             int cols = 1;
             while (2 * cols * T <= sqw_tile_elems<R>() && 2 * cols <= SQW_MAX_COLS &&
                    sqw_single_lds<R>(T, 2 * cols) <= SQW_MAX_LDS)
                 cols *= 2;
             const int ev = tm.begin(ST_REDUCE, st);
-            launch_sqw_single<R>(p, rpT, cols, amp, twT.as<Cx<R>>(), win_d.as<double>(), r->d_qfac, d_S, d_Stot, st);
+            launch_sqw_single<R>(p, rp, cols, amp, tw, win_d, r->d_qfac, d_S, d_Stot, st);
             tm.end(ev, st);
         } else if (p.n_frame == 1) {
             // one window: a DFT sum per frequency
-            dft_twiddles(p.n_int, st);
+            const Cx<double> *tw = dft_twiddles(p.n_int, st);
             const int ev = tm.begin(ST_REDUCE, st);
-            launch_sqw_window1<R>(p, amp, r->d_qfac, win_d.as<double>(), twN.as<double2>(), d_S, d_Stot, st);
+            launch_sqw_window1<R>(p, amp, r->d_qfac, win_d, tw, d_S, d_Stot, st);
             tm.end(ev, st);
         } else {
-            dft_twiddles(p.n_int, st);
-            hann_table(T, p.n_int, p.win_kind, st);
+            const Cx<double> *tw = dft_twiddles(p.n_int, st), *hn = hann_table(T, p.n_int, p.win_kind, st);
             const int ev = tm.begin(ST_REDUCE, st);
-            launch_sqw_sliding<R>(p, amp, r->d_qfac, twN.as<double2>(), hann.as<double2>(), d_S, d_Stot, st);
+            launch_sqw_sliding<R>(p, amp, r->d_qfac, tw, hn, d_S, d_Stot, st);
             tm.end(ev, st);
         }
         HIPCHK(hipGetLastError());

@@ -2,6 +2,8 @@
 // includer brings the HIP runtime's declarations and the MPSQ_ERR_* codes.
 #pragma once
 #include <algorithm>
+#include <array>
+#include <cstdint>
 #include <cstring>
 #include <vector>
 
@@ -49,6 +51,30 @@ struct DevBuf {
     }
     template <typename T> T *as() const { return static_cast<T *>(p); }
     ~DevBuf() { release(); }
+};
+
+// A device table made from a few numbers (its key), uploaded again when they
+// change.  The key is dropped first, so that a table whose allocation fails is
+// made anew by the next call and not taken for the old one.
+template <typename T> struct KeyedTable {
+    DevBuf d;
+    std::vector<T> h;
+    std::array<int64_t, 3> key{};
+    bool valid = false;
+    // fill: writes the n entries
+    template <typename F> const T *get(const std::array<int64_t, 3> &k, size_t n, hipStream_t st, F fill)
+    {
+        if (!valid || key != k) {
+            valid = false;
+            h.assign(n, T{});
+            fill(h.data());
+            d.ensure(sizeof(T) * n);
+            HIPCHK(hipMemcpyAsync(d.p, h.data(), sizeof(T) * n, hipMemcpyHostToDevice, st));
+            key = k;
+            valid = true;
+        }
+        return d.template as<T>();
+    }
 };
 
 // ---------------------------------------------------------------------------

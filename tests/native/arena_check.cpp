@@ -1,4 +1,4 @@
-// Host check of the job tables (mpsq_buffers.h, Arena) over a stand-in for the
+// Host check of the job tables and keyed tables (mpsq_buffers.h) over a stand-in for the
 // HIP runtime whose "device" is host memory: equal tables are not uploaded
 // again, changed ones are, and after a fill that was cut short by a failed
 // allocation the device still ends with the tables of the next run.  Prints
@@ -106,6 +106,28 @@ int main()
         fail_dev = -1;
         CHECK(fill(A, big, s1) && same(A, big));
         CHECK(fill(A, a, s1) && same(A, a));
+    }
+    {
+        // a table whose allocation failed is made anew, not taken for the old one
+        KeyedTable<int> K;
+        auto get = [&](int v, size_t n) -> const int * {
+            try {
+                return K.get({v, 0, 0}, n, s1, [&](int *h) { std::fill(h, h + n, v); });
+            } catch (const Err &) {
+                return nullptr;
+            }
+        };
+        const int *p = get(3, 10);
+        const int n0 = copies;
+        CHECK(p && p[0] == 3 && p[9] == 3);
+        CHECK(get(3, 10) == p && copies == n0);
+        fail_dev = 0;
+        CHECK(!get(4, 1000));
+        fail_dev = -1;
+        p = get(3, 10);
+        CHECK(p && p[0] == 3 && p[9] == 3);
+        p = get(4, 1000);
+        CHECK(p && p[999] == 4);
     }
     std::printf("ok\n");
     return 0;
