@@ -2131,15 +2131,13 @@ static void dos_run(const float *d_vel, int64_t T, int64_t n_tot, const int32_t 
     if (single) {
         std::vector<Cx<R>> twh;
         upload_twiddles<R>(tw, (int)T, st, twh);
-        while (2 * cols * T <= sqw_tile_elems<R>() && 2 * cols <= SQW_MAX_COLS &&
-               dos_fused_lds<R>(T, 2 * cols) <= SQW_MAX_LDS)
-            cols *= 2;
+        cols = dos_fused_cols<R>(T, ncs);
     }
     launch_zero_i32(reinterpret_cast<int *>(d_dos), (int)(2 * n_freq * nsp), st);
     if (single) {
         // one pass: FFT, |X|^2 and per-block species sums (no |FFT|^2 rows in HBM)
         const int64_t nout = (int64_t)nsp * n_freq;
-        const int64_t rows = dos_fused_rows<R>((ncs + cols - 1) / cols, n_freq);
+        const int64_t rows = dos_fused_rows<R>(ncs, cols, nout);
         DevBuf part;
         part.ensure(sizeof(double) * (size_t)((rows + dos_reduce_groups()) * nout));
         DosParams dp{};

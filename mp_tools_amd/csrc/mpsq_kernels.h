@@ -162,6 +162,7 @@ template <typename R> struct ColJob {
 // S(Q,w) reduction parameters
 // Q columns of one k_sqw_single workgroup: a power of two <= this
 constexpr int SQW_MAX_COLS = 64;
+constexpr int DOS_MAX_COLS = 512;  // threads of its workgroup
 
 struct SqwParams {
     int64_t T, NQ;      // frames; modes reduced (outputs [n_f][NQ], [NQ])
@@ -321,7 +322,7 @@ void launch_dos_species(const double *S, int64_t ncols, int64_t c0, int64_t n_fr
                         double *dos, hipStream_t st);
 void launch_cols_to_f64(const float *in, int64_t T, int64_t ncs, int64_t c0, int64_t nc, double *out, hipStream_t st);
 // mp_dos spectra in one pass: time FFT of packed velocity columns
-// [c0, c0 + nc) (ncs per frame) and per-block species sums part[row][s][f];
+// [c0, c0 + nc) (ncs per frame) and per-block species sums part[block][s][f];
 // dos_reduce_parts adds nrows such rows into dos[f][s] in a fixed order
 // (part2: dos_reduce_groups() * nsp * n_freq doubles)
 struct DosParams {
@@ -333,9 +334,11 @@ template <typename R> size_t dos_fused_lds(int64_t T, int cols);
 template <typename R>
 void launch_dos_fused(const DosParams &p, const RadixPlan &rp, int cols, const float *vel, const int *at_ind,
                       const typename cplx<R>::T *tw, const double *win, double *part, hipStream_t st);
-// rows of part (nsp * n_freq sums each) a launch over `groups` groups of columns
-// writes, and whether its threads hold the sums of n_freq frequencies
-template <typename R> int64_t dos_fused_rows(int64_t groups, int64_t n_freq);
+// columns per group for ncs columns of T frames, the rows of part (nout = nsp *
+// n_freq sums each) a launch over them writes, and whether its threads hold the
+// sums of n_freq frequencies
+template <typename R> int dos_fused_cols(int64_t T, int64_t ncs);
+template <typename R> int64_t dos_fused_rows(int64_t ncs, int cols, int64_t nout);
 template <typename R> bool dos_fused_ok(int64_t n_freq);
 int dos_reduce_groups();
 void dos_reduce_parts(const double *part, int64_t nrows, int nsp, int n_freq, double *part2, double *dos,

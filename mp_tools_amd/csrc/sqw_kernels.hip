@@ -746,14 +746,18 @@ template <typename C> __device__ __forceinline__ void pin(C &v) { asm volatile("
 //   (|X(f)|^2 + |X(-f)|^2) / 2 * norm
 // in FP64 registers: thread (f, h) the columns h, h + nh, ..., from one that
 // depends on f so that lanes read different LDS banks (nh = NT / n_freq
-// shares of the columns; beyond NT frequencies a thread holds several).  The
-// sums belong to the atom type the columns are of; when it changes (groups of
-// several types: for each in turn) they go to the row of share h,
-// part[block * nh + h][type][f], and start again.  dos_reduce_parts adds the
-// rows in a fixed order.  At most 128 registers: two workgroups per CU.
+// shares of the columns, no more than there are columns; beyond NT frequencies
+// a thread holds several).  The sums belong to the one type the groups so far
+// were of; when it changes, the shares are added in LDS, and the thread that
+// owns (type, f) adds them to the block's row part[block][type][f].  A group
+// of several types goes to the row directly: its columns are put in order of
+// their types, and the owner of (type, f) adds those of its type.  dos_reduce_parts adds the rows in a fixed order.  At
+// most 128 registers: two workgroups per CU.
 // (640,000 columns of 512 frames, 5 types x 256 frequencies, with a row per
 // group and a test of every column per type and frequency: 2 x 841 us and 2 x
-// 131 us for its 410 MB of rows; now 1584 us in one launch.)
+// 131 us for its 410 MB of rows; now 1584 us in one launch.  20 frames of 40,000
+// atoms, calls with their allocations: 83 us so, 216 with a row per share, 58 now;
+// 200 frames whose types alternate atom by atom 200, 230, 178.)
 // KO: frequencies per thread (1 while n_freq <= NT)
 constexpr int DOS_ACC = 9;
 template <typename R, int E, int NT, int KO>
@@ -768,28 +772,43 @@ __global__ __launch_bounds__(NT, 4) void k_dos_fused(DosParams p, RadixPlan rp, 
     const int T = (int)p.T;
     C *tile = reinterpret_cast<C *>(smem_raw);  // [T][cols]
     C *tw_l = tile + T * cols;
-    __shared__ int spc[SQW_MAX_COLS];
+    __shared__ int spc[DOS_MAX_COLS];
+    __shared__ short lst[DOS_MAX_COLS], tlo[64], thi[64];
+    __shared__ double comb[NT];
     for (int i = threadIdx.x; i < T; i += NT) tw_l[i] = tw[i];
-    const int nf = (int)p.n_freq, nout = p.nsp * nf;
+    const int nf = (int)p.n_freq, nout = p.nsp * nf, lane = threadIdx.x & 63;
     const int h = nh > 1 ? (int)fdiv((uint32_t)threadIdx.x, dnf) : 0;
     const int f0 = (int)threadIdx.x - h * nf;  // first frequency (nh == 1: then every NT-th)
     const bool own = h < nh && f0 < nf;
     const int ns = own ? (cols - h + nh - 1) / nh : 0;  // columns of the share in a whole group
     const int rot = ns > 0 ? f0 % ns : 0;
-    double *row = part + (int64_t)(blockIdx.x * nh + h) * nout;
+    double *row = part + (int64_t)blockIdx.x * nout;  // entry i belongs to thread i mod NT
     double acc[KO];
 #pragma unroll
     for (int k = 0; k < KO; ++k) acc[k] = 0.0;
-    if (own)
-        for (int f = f0; f < nf; f += NT)
-            for (int s = 0; s < p.nsp; ++s) row[s * nf + f] = 0.0;
-    int cur = -1;  // type the sums are of
+    for (int i = threadIdx.x; i < nout; i += NT) row[i] = 0.0;
+    const double sc = 0.5 * p.norm;
+    int cur = -1;  // type the sums are of (uniform)
+    // every thread of the block calls it (barriers)
     auto flush = [&]() {
+        if (cur < 0) return;
 #pragma unroll
         for (int k = 0; k < KO; ++k) {
-            const int f = f0 + k * NT;
-            if (own && f < nf && cur >= 0) row[cur * nf + f] += acc[k] * (0.5 * p.norm);
+            if (k * NT >= nf) break;  // uniform
+            if (own) comb[threadIdx.x] = acc[k];
             acc[k] = 0.0;
+            __syncthreads();
+            for (int o = nh; o > 1;) {  // share h takes share h + half, so that share 0 ends with the sum
+                const int half = (o + 1) >> 1;
+                if (own && h + half < o) comb[threadIdx.x] += comb[threadIdx.x + half * nf];
+                __syncthreads();
+                o = half;
+            }
+            // the owners of (cur, f), f in [k NT, k NT + NT)
+            const int n = min(nf - k * NT, NT), b = cur * nf + k * NT;
+            const int x = (int)((threadIdx.x + NT - (unsigned)b % NT) % NT);
+            if (x < n) row[b + x] += comb[x] * sc;
+            __syncthreads();
         }
     };
     for (int g = blockIdx.x; g < ngroups; g += gridDim.x) {
@@ -827,46 +846,80 @@ __global__ __launch_bounds__(NT, 4) void k_dos_fused(DosParams p, RadixPlan rp, 
         }
         __syncthreads();
         lds_fft<C, E>(tile, rp, cols, dcols, cols, 1, tw_l, true, tid, done);
-        // the group's types, each after the one before it in column order
-        for (int cs = 0; cs < ncol;) {
-            const int s = __builtin_amdgcn_readfirstlane(spc[cs]);
-            int ce = cs + 1;  // columns [cs, ce) are of type s
-            while (ce < ncol && __builtin_amdgcn_readfirstlane(spc[ce]) == s) ++ce;
-            if (s >= 0) {
-                if (s != cur) {
-                    flush();
-                    cur = s;
-                }
-                if (own) {
+        auto power = [&](int f, int c) -> double {
+            const C a = tile[f * cols + c], b = tile[(f == 0 ? 0 : T - f) * cols + c];
+            return ((double)a.x * (double)a.x + (double)a.y * (double)a.y) +
+                   ((double)b.x * (double)b.x + (double)b.y * (double)b.y);
+        };
+        const int s0 = __builtin_amdgcn_readfirstlane(spc[0]);
+        bool one = true;  // a whole group of one type (uniform)
+        for (int c = lane; c - lane < cols; c += 64) one = one && __all(c >= cols || spc[c] == s0);
+        if (one && s0 >= 0) {
+            if (s0 != cur) {
+                flush();
+                cur = s0;
+            }
+            if (own) {
 #pragma unroll
-                    for (int k = 0; k < KO; ++k) {
-                        const int f = f0 + k * NT;
-                        if (k * NT >= nf) break;  // uniform
-                        if (f >= nf) continue;
-                        const C *ta = tile + f * cols, *tb = tile + (f == 0 ? 0 : T - f) * cols;
-                        double x = acc[k];
-                        auto add = [&](int c) {
-                            const C a = ta[c], b = tb[c];
-                            x += ((double)a.x * (double)a.x + (double)a.y * (double)a.y) +
-                                 ((double)b.x * (double)b.x + (double)b.y * (double)b.y);
-                        };
-                        if (ce - cs == cols) {
-                            // a whole group: lane f starts at column f mod ns of
-                            // its share (rows are a multiple of the banks apart)
-                            int i = rot;
+                for (int k = 0; k < KO; ++k) {
+                    const int f = f0 + k * NT;
+                    if (k * NT >= nf) break;  // uniform
+                    if (f >= nf) continue;
+                    double x = acc[k];
+                    // lane f starts at column f mod ns of its share (rows are
+                    // a multiple of the banks apart)
+                    int i = rot;
 #pragma unroll 4
-                            for (int n = 0; n < ns; ++n) {
-                                add(h + i * nh);
-                                if (++i == ns) i = 0;
-                            }
-                        } else {
-                            for (int c = cs + h; c < ce; c += nh) add(c);
-                        }
-                        acc[k] = x;
+                    for (int n = 0; n < ns; ++n) {
+                        x += power(f, h + i * nh);
+                        if (++i == ns) i = 0;
                     }
+                    acc[k] = x;
                 }
             }
-            cs = ce;
+        } else if (!one) {
+            // the columns in order of their types (in place), then, 64 types at
+            // a time, where each type's columns begin and end
+            int s = -1, r = 0;
+            if (tid < cols) {
+                s = spc[tid];
+                for (int c = 0; c < cols; ++c) {
+                    const int q = spc[c];
+                    r += (q < s || (q == s && c < tid)) ? 1 : 0;
+                }
+            }
+            __syncthreads();
+            if (tid < cols) {
+                spc[r] = s;
+                lst[r] = (short)tid;
+            }
+            for (int sb = 0; sb < p.nsp; sb += 64) {
+                if (tid < 64) tlo[tid] = thi[tid] = 0;
+                __syncthreads();
+                if (tid < cols) {
+                    const int q = spc[tid], b = q - sb;
+                    if (b >= 0 && b < 64) {
+                        if (tid == 0 || spc[tid - 1] != q) tlo[b] = (short)tid;
+                        if (tid == cols - 1 || spc[tid + 1] != q) thi[b] = (short)(tid + 1);
+                    }
+                }
+                __syncthreads();
+                const int i0 = sb * nf, i1 = min(p.nsp, sb + 64) * nf;
+                // first entry of the window that this thread owns
+                for (int i = i0 + (int)((threadIdx.x + NT - (unsigned)i0 % NT) % NT); i < i1; i += NT) {
+                    const int b = i / nf - sb, f = i - (b + sb) * nf;
+                    const int lo = tlo[b], cnt = thi[b] - lo;
+                    if (cnt == 0) continue;
+                    int j = f % cnt;
+                    double x = 0.0;
+                    for (int n = 0; n < cnt; ++n) {
+                        x += power(f, lst[lo + j]);
+                        if (++j == cnt) j = 0;
+                    }
+                    row[i] += x * sc;
+                }
+                __syncthreads();
+            }
         }
         __syncthreads();
     }
@@ -879,19 +932,38 @@ template <typename R> size_t dos_fused_lds(int64_t T, int cols)
 }
 
 // shares of the columns: threads per frequency
-template <typename R> static int dos_shares(int64_t n_freq)
+template <typename R> static int dos_shares(int64_t n_freq, int cols)
 {
-    return (int)std::max<int64_t>(1, SqwTiles<R>::NT / n_freq);
+    return (int)std::min<int64_t>(cols, std::max<int64_t>(1, SqwTiles<R>::NT / n_freq));
 }
 
-// rows of part a launch over `groups` column groups writes
-template <typename R> int64_t dos_fused_rows(int64_t groups, int64_t n_freq)
+static int dos_cus()
 {
     int dev = 0, ncu = 0;
     (void)hipGetDevice(&dev);
     (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-    // two workgroups per CU by the LDS of their tiles
-    return std::min<int64_t>(groups, 2 * std::max(1, ncu)) * dos_shares<R>(n_freq);
+    return std::max(1, ncu);
+}
+
+// Columns per group of ncs columns of T frames: the most whose tile the
+// threads hold, up to 64, and beyond that (short series) while two groups per
+// CU are left.
+template <typename R> int dos_fused_cols(int64_t T, int64_t ncs)
+{
+    const int64_t two = 2 * dos_cus();
+    int cols = 1;
+    while (2 * cols * T <= sqw_tile_elems<R>() && 2 * cols <= DOS_MAX_COLS && dos_fused_lds<R>(T, 2 * cols) <= SQW_MAX_LDS &&
+           (2 * cols <= SQW_MAX_COLS || ncs / (2 * cols) >= two))
+        cols *= 2;
+    return cols;
+}
+
+// Workgroups, each with a row of nout sums: two per CU (by their registers, and
+// by the LDS of whole tiles), and rows within 256 MB.
+template <typename R> int64_t dos_fused_rows(int64_t ncs, int cols, int64_t nout)
+{
+    const int64_t most = std::max<int64_t>(1, ((int64_t)256 << 20) / (8 * nout));
+    return std::min<int64_t>({(ncs + cols - 1) / cols, 2 * dos_cus(), most});
 }
 
 template <typename R> bool dos_fused_ok(int64_t n_freq) { return n_freq <= (int64_t)DOS_ACC * SqwTiles<R>::NT; }
@@ -902,7 +974,7 @@ void launch_dos_fused(const DosParams &p, const RadixPlan &rp, int cols, const f
 {
     constexpr int E = SqwTiles<R>::E, NT = SqwTiles<R>::NT;
     const int64_t ng = (p.nc + cols - 1) / cols;
-    const int nh = dos_shares<R>(p.n_freq);
+    const int nh = dos_shares<R>(p.n_freq, cols);
     // set once per process (a function-local static initialises thread-safely)
     static const bool attr = [] {
         for (const void *fn : {reinterpret_cast<const void *>(&k_dos_fused<R, E, NT, 1>),
@@ -911,7 +983,7 @@ void launch_dos_fused(const DosParams &p, const RadixPlan &rp, int cols, const f
         return true;
     }();
     (void)attr;
-    const dim3 grid((unsigned)(dos_fused_rows<R>(ng, p.n_freq) / nh));
+    const dim3 grid((unsigned)dos_fused_rows<R>(p.nc, cols, (int64_t)p.nsp * p.n_freq));
     const size_t lds = dos_fused_lds<R>(p.T, cols);
     const FDiv dc = make_fdiv((uint32_t)cols), df = make_fdiv((uint32_t)p.n_freq);
     const float2 *v = reinterpret_cast<const float2 *>(vel);
@@ -932,6 +1004,7 @@ __global__ void k_dos_groups(const double *__restrict__ part, int64_t nrows, int
     if (i >= nout) return;
     const int64_t r0 = (int64_t)blockIdx.y * per, r1 = min(r0 + per, nrows);
     double s = 0.0;
+#pragma unroll 8
     for (int64_t r = r0; r < r1; ++r) s += part[r * nout + i];
     part2[(int64_t)blockIdx.y * nout + i] = s;
 }
@@ -942,6 +1015,7 @@ __global__ void k_dos_final(const double *__restrict__ part2, int ng, int nsp, i
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nsp * n_freq) return;
     double s = 0.0;
+#pragma unroll 8
     for (int g = 0; g < ng; ++g) s += part2[(int64_t)g * nsp * n_freq + i];
     const int sp = i / n_freq, f = i - sp * n_freq;
     dos[(int64_t)f * nsp + sp] += s;
@@ -952,8 +1026,10 @@ int dos_reduce_groups() { return 64; }
 void dos_reduce_parts(const double *part, int64_t nrows, int nsp, int n_freq, double *part2, double *dos,
                       hipStream_t st)
 {
-    const int nout = nsp * n_freq, G = dos_reduce_groups();
-    const int64_t per = (nrows + G - 1) / G;
+    const int nout = nsp * n_freq;
+    // about as many rows per group as groups: the two chains of adds are shortest
+    int64_t per = std::max<int64_t>(1, (nrows + dos_reduce_groups() - 1) / dos_reduce_groups());
+    while (per * per < nrows) ++per;
     const int ng = (int)((nrows + per - 1) / per);
     hipLaunchKernelGGL(k_dos_groups, dim3((unsigned)((nout + 255) / 256), (unsigned)ng), dim3(256), 0, st, part, nrows,
                        per, nout, part2);
@@ -1020,7 +1096,8 @@ void launch_sqw_single(const SqwParams &p, const RadixPlan &rp, int cols, const 
     template void launch_iqt<R>(const SqwParams &, const cplx<R>::T *, const float *, double *, double *, hipStream_t); \
     template void launch_iqt_fft<R>(const SqwParams &, const RadixPlan &, int, const cplx<R>::T *, const double2 *,  \
                                     const float *, double *, double *, hipStream_t);                                 \
-    template int64_t dos_fused_rows<R>(int64_t, int64_t);                                                             \
+    template int dos_fused_cols<R>(int64_t, int64_t);                                                                 \
+    template int64_t dos_fused_rows<R>(int64_t, int, int64_t);                                                        \
     template bool dos_fused_ok<R>(int64_t);                                                                           \
     template size_t dos_fused_lds<R>(int64_t, int);                                                                   \
     template void launch_dos_fused<R>(const DosParams &, const RadixPlan &, int, const float *, const int *,          \
