@@ -983,6 +983,37 @@ __global__ __launch_bounds__(NarrowCfg::NT, 4) void k_spread_narrow(const Spread
 // call; a 10.5 M atom frame to 512 x 512 x 64 in FP32, whose tiles are all
 // queued: 9.94 -> 5.80 ms.)
 // ---------------------------------------------------------------------------
+// LDS cycles of one 8-byte atomic add of a wave whose lane is on cell `cell`:
+// 2 (integers 1) for each lane on the fullest of 16 slots of 8 bytes, whichever
+// lanes these are, and 1 more for each lane there whose address a lower lane
+// has (measured, FP64: lanes 1 cell apart 8 cycles, 8 cells 64, 16 cells 128,
+// all on one cell 191).  Addresses are told apart by 10 bits.
+template <bool F64> __device__ __forceinline__ int add_cycles(int cell, bool have)
+{
+    unsigned long long same = __ballot(have), slot = 0;
+#pragma unroll
+    for (int b = 0; b < 10; ++b) {
+        const bool one = (cell >> b) & 1;
+        const unsigned long long bal = __ballot(one);
+        same &= one ? bal : ~bal;
+        if (b == 3) slot = same;
+    }
+    const unsigned long long later = __ballot(have && (same & ((1ull << (threadIdx.x & 63)) - 1ull)) != 0ull);
+    const int n = have ? (F64 ? 2 : 1) * __popcll(slot) + __popcll(slot & later) : 0;
+    // the largest over the lanes
+    int most = 0;
+    unsigned long long top = ~0ull;
+#pragma unroll
+    for (int b = 7; b >= 0; --b) {
+        const unsigned long long bal = __ballot((n >> b) & 1) & top;
+        if (bal) {
+            most |= 1 << b;
+            top = bal;
+        }
+    }
+    return most;
+}
+
 struct PassRect {
     int y0, z0, by, bz;  // rows of the pass: by x bz from (y0, z0)
 };
@@ -1016,14 +1047,16 @@ __global__ __launch_bounds__(512, 4) void k_spread_wide(const SpreadJob<R> *__re
     const int xbeg = fbl ? 0 : xr[xcd], xend = fbl ? wc[CTR_FB_COUNT] : xr[xcd + 1];
     unsigned long long *acc64 = reinterpret_cast<unsigned long long *>(smem_raw + narrow_bias(W));
     double *accd = reinterpret_cast<double *>(smem_raw + narrow_bias(W));
-    // lane order of a stencil's cells: rotated by lane group as in the narrow
-    // kernel (8-byte cells; a 10.5 M atom crystal to 512 x 512 x 64 in FP32
-    // 4.75 -> 3.36 ms a call, 320,000 atoms x 16 frames in FP64 4.30 -> 4.0)
+    // Lane order of a stencil's cells: as they lie, or rotated by lane group as
+    // in the narrow kernel, as the lanes' cells then collide less: a wave looks
+    // at its first points of one pass in 64.  Lattices have lanes a fixed step
+    // apart, and whether the rotation spreads or piles them depends on that
+    // step: at 8 cells (10.5 M atoms to 512 x 512 x 64, FP32) the launch takes
+    // 3.56 ms as they lie, 2.20 rotated and 2.21 so; at 6 cells (33 x 33 x 33
+    // unit cells x 16 frames to 100 x 120 x 32, FP64, complex) 1.92, 5.32, 1.96.
     constexpr int NG = (W >= 4) ? 4 : (W >= 2 ? 2 : 1), RSTEP = W / NG;
-    const int rg = lane & (NG - 1), rot = rg * RSTEP;
-    int rofs[NG];
-#pragma unroll
-    for (int s = 0; s < NG; ++s) rofs[s] = 8 * rot - ((rg >= NG - s) ? 8 * W : 0);
+    int rmask = 0;  // of the lane's group: 0 as they lie, NG - 1 rotated (uniform)
+    int look = 0;   // passes until the wave looks again
     C *tile = reinterpret_cast<C *>(smem_raw);
     // next item: its position k in [xbeg, xend) (k >= xend: none) -> tile id, pass
     auto take = [&]() -> int {
@@ -1106,6 +1139,21 @@ __global__ __launch_bounds__(512, 4) void k_spread_wide(const SpreadJob<R> *__re
             finv = ldexp(1.0, -qq);
         }
 
+        if (look <= 0 && vw < total) {  // the wave's first points of the pass (uniform)
+            const int a = __mul24(__mul24(cd.pr.lz, P.by) + cd.pr.ly, RS) + cd.pr.lx;
+            // rotated if that is clearly cheaper, at the first cells and where
+            // some groups have wrapped (as they lie, every cell is the same)
+            const int lies = add_cycles<!F32>(a, cd.have), r = (lane & (NG - 1)) * RSTEP;
+            const int t0 = add_cycles<!F32>(a + r, cd.have);
+            rmask = 0;
+            if (8 * t0 < 7 * lies && 4 * (t0 + add_cycles<!F32>(a + (r + W - 2) % W, cd.have)) < 7 * lies)
+                rmask = NG - 1;
+            look = 64;
+        }
+        const int rg = lane & rmask, rot = rg * RSTEP;
+        int rofs[NG];
+#pragma unroll
+        for (int s = 0; s < NG; ++s) rofs[s] = 8 * rot - ((rg >= NG - s) ? 8 * W : 0);
         for (int v0 = vw; v0 < total; v0 += NT) {
             const PtRec<R> p = cd.pr;
             const C cc = cd.cv;
@@ -1272,6 +1320,7 @@ __global__ __launch_bounds__(512, 4) void k_spread_wide(const SpreadJob<R> *__re
         __syncthreads();  // every read of the tile (and the twiddles) done
         if (jn != j) load_twiddles<R, NT>(jobs[jn], smem_raw, jobs[jn].lds_tw);
         pb ^= 1;
+        look = jn == j ? look - 1 : 0;
         j = jn;
         t = tn;
         P = Pn;
