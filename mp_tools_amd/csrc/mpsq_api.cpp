@@ -1210,11 +1210,26 @@ template <typename R> struct Engine {
             return;
         }
         RadixPlan rp{};
-        // one window: direct DFT sums where they are fewer than the LDS FFT's
-        // fixed work (2.1 M columns, FP32: 16 frames to 8 frequencies 136 us
-        // against 348, 24 to 12 263 against 390, 32 to 16 388 against 407, 24
-        // to 24 426 against 420; FP64 alike), or none (S_tot alone)
-        const bool direct = p.n_f == 0 || T * p.n_f <= 400;
+        // One window: direct DFT sums (FP64) where they take less than the LDS
+        // FFT, or none (S_tot alone).  Measured over 1 to 512 frames, 0 to 32
+        // frequencies, 128 to 2.1 M columns, both precisions (us direct / FFT):
+        //  many columns: the FFT's fixed work is the larger up to about 384
+        //   products (2.1 M columns, FP32: 16 frames to 8 frequencies 132 / 338,
+        //   24 to 16 284 / 401, 32 to 16 350 / 408, 24 to 24 405 / 412, 20 to 20
+        //   437 / 372), but for the 64-point FFT in FP64 (64 frames to 4: 736 /
+        //   637, 48 to 8: 543 / 616, 100 to 2: 1188 / 1316);
+        //  few: launches and the walk of a wave over its frames, whatever the
+        //   frequencies (4,096 columns, FP32: 20 frames to 20 17 / 18, 100 to 4
+        //   21 / 22, 200 to 2 28 / 23, 400 to 1 44 / 24; FP64: 64 to 4 19 / 20,
+        //   128 to 1 23 / 21);
+        //  between: both (25,600 columns, FP32: 20 frames to 12 19 / 19, to 20 22
+        //   / 20, 100 to 4 23 / 25, 200 to 2 41 / 38; FP64: 400 to 1 74 / 89).
+        const int64_t prod = T * p.n_f;
+        const bool f32 = sizeof(R) == 4;
+        const bool direct = p.n_f == 0 ? true
+                            : p.NQ < 8192 ? prod <= 400 && T <= (f32 ? 100 : 64)
+                            : p.NQ < 131072 ? (prod <= 240 && T <= 48) || (prod <= 400 && p.n_f <= 4 && T <= (f32 ? 128 : 400))
+                                            : prod <= 384 && (f32 || T <= 48 || T >= 100);
         const bool single = (p.n_frame == 1) && !direct && (T <= sqw_tile_elems<R>()) &&
                             sqw_single_lds<R>(T, 1) <= SQW_MAX_LDS && radix_plan((int)T, rp);
         const double *win_d = nullptr;
