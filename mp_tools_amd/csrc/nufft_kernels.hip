@@ -549,6 +549,53 @@ __device__ __forceinline__ int xcd_block(int b, int nb)
     return x * q + min(x, r) + (b >> 3);
 }
 
+constexpr int COLFFT_NT_FINAL[] = {256, 512, 1024};  // threads of the final pass
+
+// Output kk of column c of a final pass, to the map.  herm: column col = km *
+// hH1 + kh (3D; 2D: col = kh); the transformed axis' index kk.  Mode (kk, km,
+// kh) goes to its place and, when k1 < 0, its mirror (2 h - kk, 2 h2 - km, 2 h1 -
+// kh), where in range, as the conjugate: every mode of the map is written once.
+template <typename R> struct ColOut {
+    using CS = typename cplx<R>::T;
+    bool herm, cj, mid;
+    int N, inner, col0, N1, N2, H1, H1v, h, h1, h2;
+    int64_t hsa;
+    FDiv dH1;
+    CS *map;
+    __device__ __forceinline__ ColOut(const ColJob<R> &J, int grp, int o, int col0_)
+        : herm(J.cp.herm != 0), cj(J.cp.conj != 0), mid(J.cp.hmid != 0), N(J.cp.N), inner(J.cp.inner), col0(col0_),
+          N1(J.cp.hN1), N2(J.cp.hN2), H1(J.cp.hH1), H1v(J.cp.hH1v), h(J.cp.N / 2),
+          h1(J.cp.hN1 / 2), h2(J.cp.hN2 / 2), hsa(J.cp.hsa), dH1(J.cp.dH1)
+    {
+        map = J.out + (int64_t)grp * J.cp.out_tstride + (herm ? 0 : (int64_t)o * N * inner + col0);
+    }
+    __device__ __forceinline__ void put_full(int kk, int c, CS x) const
+    {
+        if (cj) x.y = -x.y;
+        if (kk < N) map[(int64_t)kk * inner + c] = x;
+    }
+    __device__ __forceinline__ void put_half(int kk, int c, CS x) const
+    {
+        if (cj) x.y = -x.y;
+        const int col = col0 + c;
+        int km = 0, kh = col;
+        if (mid) {
+            km = (int)fdiv((uint32_t)col, dH1);
+            kh = col - km * H1;
+        }
+        if (kh >= H1v) return;  // pad column
+        if (kk < N && km < N2) map[(int64_t)kk * hsa + (int64_t)km * N1 + kh] = x;
+        const int ka = 2 * h - kk, kmm = mid ? 2 * h2 - km : 0, kx = 2 * h1 - kh;
+        if (kh < h1 && kx < N1 && ka >= 0 && ka < N && kmm >= 0 && kmm < N2)
+            map[(int64_t)ka * hsa + (int64_t)kmm * N1 + kx] = cmk<CS>(x.x, -x.y);
+    }
+    __device__ __forceinline__ void put(int kk, int c, CS x) const
+    {
+        if (!herm) put_full(kk, c, x);
+        else put_half(kk, c, x);
+    }
+};
+
 template <typename R, typename RC, int E, int NT, bool FINAL>
 __global__ __launch_bounds__(NT) void k_colfft(const ColJob<R> *__restrict__ jobs, const int *__restrict__ blk0s,
                                                int njobs, int by_xcd)
@@ -562,7 +609,12 @@ __global__ __launch_bounds__(NT) void k_colfft(const ColJob<R> *__restrict__ job
     C *tile = reinterpret_cast<C *>(smem_raw);
     const int n = cp.n, N = cp.N, cols = cp.cols, inner = cp.inner;
     C *tw_l = tile + n * cols;  // twiddles in LDS
-    C *acc = tw_l + n;          // FINAL, nsp > 1: species sum of the kept modes, [NO][cols]
+    // FINAL: the kept modes, [NO][cols], where they are summed over species or,
+    // short columns (256 threads), leave for the map in a loop of their own
+    // (128 frames of 256 x 256 x 32 modes, FP32: 1.12 ms, 1.17 written from the
+    // loop below; 130,560 FP64 columns of 1024 rows: 3.2 ms through LDS, 1.9)
+    C *acc = tw_l + n;
+    constexpr bool VIA_LDS = FINAL && NT == COLFFT_NT_FINAL[0];
     const C *twg;
     if constexpr (sizeof(RC) == sizeof(R)) twg = reinterpret_cast<const C *>(J.tw);
     else twg = reinterpret_cast<const C *>(J.tw64);
@@ -580,36 +632,9 @@ __global__ __launch_bounds__(NT) void k_colfft(const ColJob<R> *__restrict__ job
     // extra half-spectrum output k = N - h takes that of -k (entry 0 for
     // even N; for odd N that output is never a mirror source)
     auto phi_ix = [&](int kk) { return kk < N ? kk : 0; };
-    // FINAL: output kk of column c to the map.  herm: column col = km * hH1 +
-    // kh (3D; 2D: col = kh); the transformed axis' index kk.  Mode (kk, km,
-    // kh) goes to its place and, when k1 < 0, its mirror (2 h - kk, 2 h2 - km,
-    // 2 h1 - kh), where in range, as the conjugate: every mode of the map is
-    // written once.
     // (the job's fields in registers: read through J after each store they
     // would be loaded again)
-    const bool herm = FINAL && cp.herm, cj = cp.conj != 0, mid = cp.hmid != 0;
-    const int N1 = cp.hN1, h1 = N1 / 2, N2 = cp.hN2, h2 = N2 / 2, H1 = cp.hH1, H1v = cp.hH1v;
-    const int64_t hsa = cp.hsa;
-    const FDiv dH1 = cp.dH1;
-    CS *const map = J.out + (FINAL ? (int64_t)grp * cp.out_tstride + (herm ? 0 : (int64_t)o * N * inner + col0) : 0);
-    auto emit = [&](int kk, int c, CS x) {
-        if (cj) x.y = -x.y;
-        if (!herm) {
-            if (kk < N) map[(int64_t)kk * inner + c] = x;
-            return;
-        }
-        const int col = col0 + c;
-        int km = 0, kh = col;
-        if (mid) {
-            km = (int)fdiv((uint32_t)col, dH1);
-            kh = col - km * H1;
-        }
-        if (kh >= H1v) return;  // pad column
-        if (kk < N && km < N2) map[(int64_t)kk * hsa + (int64_t)km * N1 + kh] = x;
-        const int ka = 2 * h - kk, kmm = mid ? 2 * h2 - km : 0, kx = 2 * h1 - kh;
-        if (kh < h1 && kx < N1 && ka >= 0 && ka < N && kmm >= 0 && kmm < N2)
-            map[(int64_t)ka * hsa + (int64_t)kmm * N1 + kx] = cmk<CS>(x.x, -x.y);
-    };
+    const ColOut<R> om(J, grp, o, col0);
     for (int s = 0; s < nsp; ++s) {
         const int t = FINAL ? grp * cp.nsp + s : grp;
         {
@@ -650,6 +675,18 @@ __global__ __launch_bounds__(NT) void k_colfft(const ColJob<R> *__restrict__ job
                 const C x = cscale(tile[f * cols + c], (RC)J.phinv[phi_ix(kk)]);
                 dst[(int64_t)kk * inner + c] = cmk<CS>((R)x.x, (R)x.y);
             }
+        } else if constexpr (VIA_LDS) {
+            for (int i = threadIdx.x; i < NO * cols; i += NT) {
+                const int kk = (int)fdiv((uint32_t)i, cp.dcols), c = i - kk * cols;
+                int f = kk - h;
+                if (f < 0) f += n;
+                R wv = J.phinv[phi_ix(kk)];
+                // (a half-spectrum pass has no per-Q table: the host keeps those jobs full)
+                if (J.wtab) wv *= (c < ncol) ? (R)J.wtab[(int64_t)s * cp.NQ + (int64_t)kk * inner + col0 + c] : (R)0;
+                else if (J.wsc) wv *= J.wsc[s];
+                const C x = cscale(tile[f * cols + c], wv);
+                acc[i] = (s == 0) ? x : cadd(acc[i], x);
+            }
         } else {
             const R *phinv = J.phinv;
             const float *wtab = J.wtab;
@@ -667,10 +704,25 @@ __global__ __launch_bounds__(NT) void k_colfft(const ColJob<R> *__restrict__ job
                 C x = cscale(tile[f * cols + c], wv);
                 if (s > 0) x = cadd(acc[i], x);
                 if (s + 1 < nsp) acc[i] = x;
-                else if (c < ncol) emit(kk, c, x);
+                else if (c < ncol) om.put(kk, c, x);
             }
         }
         __syncthreads();
+    }
+    if constexpr (VIA_LDS) {
+        // (its fields now: held across the FFT they spill)
+        const ColOut<R> late(J, grp, o, col0);
+        if (cp.herm) {
+            for (int i = threadIdx.x; i < NO * cols; i += NT) {
+                const int kk = (int)fdiv((uint32_t)i, cp.dcols), c = i - kk * cols;
+                if (c < ncol) late.put_half(kk, c, acc[i]);
+            }
+        } else {
+            for (int i = threadIdx.x; i < N * cols; i += NT) {
+                const int kk = (int)fdiv((uint32_t)i, cp.dcols), c = i - kk * cols;
+                if (c < ncol) late.put_full(kk, c, acc[i]);
+            }
+        }
     }
 }
 
@@ -695,7 +747,6 @@ template <typename R> struct Tiles;
 template <> struct Tiles<float> { static constexpr int EY = 8, EF = 8; using RY = float; };
 template <> struct Tiles<double> { static constexpr int EY = 4, EF = 4; using RY = double; };
 constexpr int COLFFT_NT_Y = 1024;
-constexpr int COLFFT_NT_FINAL[] = {256, 512, 1024};
 constexpr int64_t FINAL_BLOCKS = 1024;
 
 template <typename R>
@@ -824,11 +875,12 @@ template <typename R> int colfft_cols(int64_t n, int64_t inner, int64_t slabs, b
     return cols;
 }
 
-// LDS of one column pass of a job: tile + twiddles (+ species sum for the final pass)
+// LDS of one column pass of a job: tile + twiddles (+ the final pass' kept modes, see k_colfft)
 template <typename R> size_t colfft_lds(const ColPass &cp, bool final)
 {
     const size_t es = final ? sizeof(typename cplx<R>::T) : sizeof(typename cplx<typename Tiles<R>::RY>::T);
-    return ((size_t)cp.n * (cp.cols + 1) + (final && cp.nsp > 1 ? (size_t)cp.NO * cp.cols : 0)) * es;
+    const bool via = cp.nsp > 1 || cp.n * cp.cols <= Tiles<R>::EF * COLFFT_NT_FINAL[0];
+    return ((size_t)cp.n * (cp.cols + 1) + (final && via ? (size_t)cp.NO * cp.cols : 0)) * es;
 }
 
 template <typename R>
