@@ -2133,8 +2133,7 @@ static void dos_run(const float *d_vel, int64_t T, int64_t n_tot, const int32_t 
     p.norm_s = 1.0 / (double)T;
     p.norm_tot = 0.0;
     RadixPlan rp{};
-    const bool single = (T <= sqw_tile_elems<R>()) && dos_fused_lds<R>(T, 1) <= SQW_MAX_LDS && dos_fused_ok<R>(n_freq) &&
-                        radix_plan((int)T, rp);
+    const bool single = (T <= sqw_tile_elems<R>()) && dos_fused_lds<R>(T, 1) <= SQW_MAX_LDS && radix_plan((int)T, rp);
     DevBuf tw, win, S, buf;
     int cols = 1;
     std::vector<double> wh((size_t)T);
@@ -2187,11 +2186,7 @@ static void dos_run(const float *d_vel, int64_t T, int64_t n_tot, const int32_t 
             amp = reinterpret_cast<const Cx<R> *>(d_vel) + c0;
             p.NQs = ncs;
         }
-        if (single)
-            launch_sqw_single<R>(p, rp, cols, amp, tw.as<Cx<R>>(), win.as<double>(), nullptr, S.as<double>(), nullptr,
-                                 st);
-        else
-            launch_sqw_window1<R>(p, amp, nullptr, win.as<double>(), twd.as<double2>(), S.as<double>(), nullptr, st);
+        launch_sqw_window1<R>(p, amp, nullptr, win.as<double>(), twd.as<double2>(), S.as<double>(), nullptr, st);
         launch_dos_species(S.as<double>(), nc, c0, n_freq, d_at_ind, nsp, d_dos, st);
         HIPCHK(hipGetLastError());
     }

@@ -334,12 +334,10 @@ template <typename R> size_t dos_fused_lds(int64_t T, int cols);
 template <typename R>
 void launch_dos_fused(const DosParams &p, const RadixPlan &rp, int cols, const float *vel, const int *at_ind,
                       const typename cplx<R>::T *tw, const double *win, double *part, hipStream_t st);
-// columns per group for ncs columns of T frames, the rows of part (nout = nsp *
-// n_freq sums each) a launch over them writes, and whether its threads hold the
-// sums of n_freq frequencies
+// columns per group for ncs columns of T frames, and the rows of part (nout =
+// nsp * n_freq sums each) a launch over them writes
 template <typename R> int dos_fused_cols(int64_t T, int64_t ncs);
 template <typename R> int64_t dos_fused_rows(int64_t ncs, int cols, int64_t nout);
-template <typename R> bool dos_fused_ok(int64_t n_freq);
 int dos_reduce_groups();
 void dos_reduce_parts(const double *part, int64_t nrows, int nsp, int n_freq, double *part2, double *dos,
                       hipStream_t st);

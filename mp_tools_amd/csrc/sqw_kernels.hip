@@ -759,7 +759,8 @@ template <typename C> __device__ __forceinline__ void pin(C &v) { asm volatile("
 // 131 us for its 410 MB of rows; now 1584 us in one launch.  20 frames of 40,000
 // atoms, calls with their allocations: 83 us so, 216 with a row per share, 58 now;
 // 200 frames whose types alternate atom by atom 200, 230, 178.)
-// KO: frequencies per thread (1 while n_freq <= NT)
+// KO: frequencies per thread (1 while n_freq <= NT; a tile's longest series has E
+// NT / 2 + 1)
 constexpr int DOS_ACC = 9;
 template <typename R, int E, int NT, int KO>
 __global__ __launch_bounds__(NT, 4) void k_dos_fused(DosParams p, RadixPlan rp, int cols, FDiv dcols, FDiv dnf, int nh,
@@ -967,13 +968,12 @@ template <typename R> int64_t dos_fused_rows(int64_t ncs, int cols, int64_t nout
     return std::min<int64_t>({(ncs + cols - 1) / cols, 2 * dos_cus(), most});
 }
 
-template <typename R> bool dos_fused_ok(int64_t n_freq) { return n_freq <= (int64_t)DOS_ACC * SqwTiles<R>::NT; }
-
 template <typename R>
 void launch_dos_fused(const DosParams &p, const RadixPlan &rp, int cols, const float *vel, const int *at_ind,
                       const typename cplx<R>::T *tw, const double *win, double *part, hipStream_t st)
 {
     constexpr int E = SqwTiles<R>::E, NT = SqwTiles<R>::NT;
+    static_assert(DOS_ACC * NT >= E * NT / 2 + 1, "a thread holds every frequency of the longest series");
     const int64_t ng = (p.nc + cols - 1) / cols;
     const int nh = dos_shares<R>(p.n_freq, cols);
     // set once per process (a function-local static initialises thread-safely)
@@ -1099,7 +1099,6 @@ void launch_sqw_single(const SqwParams &p, const RadixPlan &rp, int cols, const 
                                     const float *, double *, double *, hipStream_t);                                 \
     template int dos_fused_cols<R>(int64_t, int64_t);                                                                 \
     template int64_t dos_fused_rows<R>(int64_t, int, int64_t);                                                        \
-    template bool dos_fused_ok<R>(int64_t);                                                                           \
     template size_t dos_fused_lds<R>(int64_t, int);                                                                   \
     template void launch_dos_fused<R>(const DosParams &, const RadixPlan &, int, const float *, const int *,          \
                                       const cplx<R>::T *, const double *, double *, hipStream_t);
