@@ -712,7 +712,7 @@ template <typename R> struct Plan {
                         binstart.as<int64_t>(), c.st);
         if (sizeof(R) == 4) {
             launch_binmax<R>(srec.as<PtRec<R>>(), binstart.as<int64_t>(), sort_tab.dev<TransformInfo>(off_tinfo), 1,
-                             c.g.nbins / c.g.BR, binmax.as<int>(), c.st);
+                             c.g.nbins / c.g.BR, M_, binmax.as<int>(), c.st);
         }
         const hipError_t le = hipGetLastError();
         HIPCHK(hipStreamSynchronize(c.st));
@@ -1533,7 +1533,8 @@ static void run_parts(const std::vector<Part<R>> &parts, Workspace<R> &ws, Arena
                     ws.binstart.template as<int64_t>(), st);
     if (sizeof(R) == 4)
         launch_binmax<R>(ws.srec.template as<PtRec<R>>(), ws.binstart.template as<int64_t>(),
-                         A.dev<TransformInfo>(o_ti), (int)ntr_all, max_bound, ws.binmax.template as<int>(), st);
+                         A.dev<TransformInfo>(o_ti), (int)ntr_all, max_bound, npts,
+                         ws.binmax.template as<int>(), st);
     tm->end(ev, st);
     ev = tm->begin(ST_SPREAD, st);
     for (const SpreadLaunch &L : sl)

@@ -227,7 +227,7 @@ size_t spread_lds_real(int rows, int n1, int w);
 // cover any one cell of a row)
 template <typename R>
 void launch_binmax(const PtRec<R> *srec, const int64_t *binstart, const TransformInfo *tinfo, int ntr, int max_nbins,
-                   int *binmax, hipStream_t st);
+                   int64_t npts, int *binmax, hipStream_t st);
 // longest column of the column passes, and the columns one workgroup takes
 // (columns of n rows, `inner` adjacent ones in each of `slabs` slabs)
 template <typename R> int colfft_max_len();

@@ -818,10 +818,15 @@ void launch_binstart(const int64_t *Hs, const TransformInfo *tinfo, int ntr, int
 
 template <typename R>
 void launch_binmax(const PtRec<R> *srec, const int64_t *binstart, const TransformInfo *tinfo, int ntr, int max_nbins,
-                   int *binmax, hipStream_t st)
+                   int64_t npts, int *binmax, hipStream_t st)
 {
     if (ntr <= 0 || max_nbins <= 0) return;
-    if ((int64_t)max_nbins * ntr < 4096)  // fewer waves than the chip holds with one per bin
+    // fewer waves than the chip holds with one per bin: a workgroup each where
+    // they are few, or hold points for 16 waves (us with a workgroup / a wave:
+    // 1,024 bins of 127 points 3.9 / 5.5, 400 of 432 4.5 / 6.0, 400 of 8,192 20 /
+    // 76, 2,400 of 83 11.0 / 5.8)
+    const int64_t bins = (int64_t)max_nbins * ntr;
+    if (bins <= 1024 || (bins < 4096 && npts >= 512 * bins))
         hipLaunchKernelGGL((k_binmax<R, 16>), dim3((unsigned)max_nbins, (unsigned)ntr), dim3(1024), 0, st, srec,
                            binstart, tinfo, binmax);
     else
@@ -927,8 +932,8 @@ void launch_colfft_jobs(const ColJob<R> *jobs, const int *blk0s, int njobs, int 
                                          const PtRec<R> *, const cplx<R>::T *, PtRec<R> *, cplx<R>::T *, int *,       \
                                          hipStream_t);                                                                \
     template void launch_gather<R>(int64_t, int, const int *, const cplx<R>::T *, cplx<R>::T *, int, hipStream_t);    \
-    template void launch_binmax<R>(const PtRec<R> *, const int64_t *, const TransformInfo *, int, int, int *,         \
-                                   hipStream_t);                                                                      \
+    template void launch_binmax<R>(const PtRec<R> *, const int64_t *, const TransformInfo *, int, int, int64_t,       \
+                                   int *, hipStream_t);                                                               \
     template int colfft_max_len<R>();                                                                                 \
     template int colfft_cols<R>(int64_t, int64_t, int64_t, bool);                                                     \
     template size_t colfft_lds<R>(const ColPass &, bool);                                                             \
