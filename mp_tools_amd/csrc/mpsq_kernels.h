@@ -300,7 +300,8 @@ struct QTableParams {
 void launch_qtables(const QTableParams &p, float *q2_norm, float *x_ffq, hipStream_t st);
 template <typename R> int sqw_tile_elems();
 // dynamic LDS of a k_sqw_single workgroup over T frames and cols Q columns;
-// launches keep it <= SQW_MAX_LDS (the kernel's own static LDS is 1 KB)
+// launches keep it <= SQW_MAX_LDS (the kernels' own static LDS is 1 KB, 8 KB in
+// k_dos_fused)
 template <typename R> size_t sqw_single_lds(int64_t T, int cols);
 constexpr size_t SQW_MAX_LDS = 150 * 1024;
 template <typename R>

@@ -103,8 +103,8 @@ template <> __host__ __device__ inline double es_shape<double>(double beta) { re
 // beta log2(e) in [6, 54].  The library's exp and sqrt handle every argument
 // (61 instructions per value with them, about three quarters of the wide FP64
 // spread's); on this range less is enough: sqrt from the hardware's reciprocal
-// root by one Newton step of the root and its half reciprocal and a residual
-// correction, 2^y as 2^n (1 + f q(f)) with n = rint(y), f = y - n exact and
+// root by one step of Goldschmidt's iteration (the root and its half reciprocal
+// together) and a residual correction, 2^y as 2^n (1 + f q(f)) with n = rint(y), f = y - n exact and
 // |f| <= 1/2, q the polynomial through (2^f - 1) / f at the 11 Chebyshev nodes
 // (2.0e-17 relative with these coefficients).  About 30 instructions.
 // (FP64 map of 320,000 atoms x 16 frames: 1.03e9 -> 0.80e9 VALU instructions

@@ -754,11 +754,12 @@ template <typename C> __device__ __forceinline__ void pin(C &v) { asm volatile("
 // were of; when it changes, the shares are added in LDS, and the thread that
 // owns (type, f) adds them to the block's row part[block][type][f].  A group
 // of several types goes to the row directly: its columns are put in order of
-// their types, and the owner of (type, f) adds those of its type.  dos_reduce_parts adds the rows in a fixed order.  At
-// most 128 registers: two workgroups per CU.
+// their types, and the owner of (type, f) adds those of its type.
+// dos_reduce_parts adds the rows in a fixed order.  At most 128 registers: two
+// workgroups per CU.
 // (640,000 columns of 512 frames, 5 types x 256 frequencies, with a row per
 // group and a test of every column per type and frequency: 2 x 841 us and 2 x
-// 131 us for its 410 MB of rows; now 1584 us in one launch.  20 frames of 40,000
+// 131 us for its 410 MB of rows; now 1501 us in one launch.  20 frames of 40,000
 // atoms, calls with their allocations: 83 us so, 216 with a row per share, 58 now;
 // 200 frames whose types alternate atom by atom 200, 230, 178.)
 // KO: frequencies per thread (1 while n_freq <= NT; a tile's longest series has E
